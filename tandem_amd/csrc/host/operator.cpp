@@ -630,8 +630,23 @@ bool Operator::uses_split() const { return variant_ == Variant_Auto && uses_mfma
 template <class T> void Operator::upload_mfma(DeviceMfma<T>& dm) {
     const unsigned D = D_, DD = D * D, NF = D + 1;
     const MfmaDims L{int(D), int(Nbf_), int(Nq_), int(nq_)};
+    // face frame: the nodes of face 0 first (their basis functions alone are nonzero there, checked), so
+    // that the kernels contract values and tangential derivatives over those nodes only
+    std::vector<unsigned> order;
+    for (int off = 0; off < 2; ++off)
+        for (unsigned k = 0; k < Nbf_; ++k) {
+            double m = 0.0;
+            for (unsigned q = 0; q < nq_; ++q) {
+                m = std::max(m, std::fabs(E_q_[0][k + Nbf_ * q]));
+                for (unsigned e = 0; e + 1 < D; ++e) m = std::max(m, std::fabs(Dxi_q_[0][k + Nbf_ * (e + D * q)]));
+            }
+            if ((m < 1e-10) == (off == 1)) order.push_back(k);
+            if (off == 0 && k + 1 == Nbf_ && order.size() != num_basis(D - 1, N_))
+                throw std::runtime_error("the basis functions off a face do not vanish on it");
+        }
     auto T0 = [&](int c, int jb, int q) -> double {
-        return c == 0 ? E_q_[0][jb + Nbf_ * q] : Dxi_q_[0][jb + Nbf_ * ((c - 1) + D * q)];
+        const unsigned k = order[std::size_t(jb)];
+        return c == 0 ? E_q_[0][k + Nbf_ * q] : Dxi_q_[0][k + Nbf_ * ((c - 1) + D * q)];
     };
     std::vector<double> V(std::size_t(D) * Nq_ * Nbf_), TT(std::size_t(NF) * nq_ * Nbf_);
     for (unsigned e = 0; e < D; ++e)
@@ -640,8 +655,13 @@ template <class T> void Operator::upload_mfma(DeviceMfma<T>& dm) {
     for (unsigned c = 0; c <= D; ++c)
         for (unsigned q = 0; q < nq_; ++q)
             for (unsigned k = 0; k < Nbf_; ++k) TT[(c * nq_ + q) * Nbf_ + k] = T0(int(c), int(k), int(q));
-    std::vector<int32_t> P2(perm_);
-    P2.insert(P2.end(), iperm_.begin(), iperm_.end());
+    std::vector<int32_t> P2(std::size_t(2) * NF * Nbf_);
+    for (unsigned f = 0; f < NF; ++f)
+        for (unsigned k = 0; k < Nbf_; ++k) {
+            const int32_t node = perm_[f * Nbf_ + order[k]];
+            P2[f * Nbf_ + k] = node;
+            P2[(NF + f) * Nbf_ + unsigned(node)] = int32_t(k);
+        }
     // element-grouped volume point data
     const std::size_t ng = (E_ + 15) / 16;
     std::vector<T> VD(ng * Nq_ * L.NCH * 16, T(0));

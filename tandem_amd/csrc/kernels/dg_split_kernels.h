@@ -23,6 +23,12 @@
 //   lifts    : Y_s(k' ; j, u) += sum_(q,c) T0(c, q ; k') W_s(c, q ; j, u)
 // and the result of side s goes to the slot L(element_s, face_s) (one 105-vector at P4 3D).
 //
+// The basis functions of the nodes off a face vanish on it: values and tangential derivatives are
+// contracted over the face's own nodes (15 of 35 at P4), only the normal derivative over all, in the
+// traces and in the lifts.  A P4 wave issues 165 MFMAs instead of 255; the apply went from 489 to
+// 450 us (FP64, 82,944 P4 tetrahedra) and 163 to 154 us (FP32, 48,000).  The kernel is then bound by
+// neither roof (FP64 matrix cores ~35% busy, ~3 TB/s) but by waits at two waves per SIMD.
+//
 // Element kernel.  One wave owns 16 consecutive elements; the volume term is the element-centric
 // kernel's (reference gradients on the matrix cores, the stress per point in registers, the
 // divergence on the matrix cores), with the accumulators started from the sum of the element's
@@ -116,6 +122,12 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
     using acc = typename Mma<T>::acc;
     constexpr int Nbf = L::Nbf, nq = L::nq, Q = D, BS = Nbf * Q, NF = D + 1, DD = D * D;
     constexpr int KS = L::KS, MT = L::MT, FT = L::FT;
+    // Trace K-steps of the four-channel tiles: the face's own nodes, and the other nodes (normal
+    // derivative only) four tiles at a time, where that spares at least 5 K-steps a wave (3D P4: 5 x 9
+    // -> 5 x 4 + 2 x 5, P3: 4 x 5 -> 4 x 3 + 2, 2D P6: 2 x 7 -> 2 x 2 + 5).  With fewer the extra pass
+    // costs more than it spares (3D P2, 2 x 3 -> 2 x 2 + 1: 28.2 -> 29.3 us at 14,586 elements, FP64).
+    constexpr bool SPLITK = (FT - (FT + 3) / 4) * (KS - L::KF) >= 5;
+    constexpr int KF = SPLITK ? L::KF : KS;
     constexpr int NFR = DD + D + 4; // tangents (D-1 columns), c_0, c_1, lam_0, mu_0, lam_1, mu_1
     constexpr int NbfP = Strides<T>::pad(Nbf), BSP = Strides<T>::pad(BS);
     constexpr int nT = NF * nq * Nbf;
@@ -217,6 +229,9 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
             const int tq = mfma_group<T>(j);
             const int tc = min(mfma_reg<T>(j), D);
             T const* const U = X + j * BSP;
+            // part of the normal derivative from the nodes off the face, four tiles at a time:
+            // register i = point 4 (4 b + i) + g of block b, this lane's point in tile 4 b + i
+            acc off[Q];
 
 #pragma unroll 1
             for (int t = 0; t < FT; ++t) {
@@ -229,38 +244,48 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
                 // values: padding facets carry the identity Jacobian, empty columns a zero vector)
                 const T wq = act ? sW[qc] : T(0);
                 const T ws = sd == 0 ? -wq : wq; // the traction term lifts with -w on side 0, +w on side 1
+                // matrix-core phases run at raised wave priority, so that the SIMD's other wave's
+                // point arithmetic fills the matrix core's busy cycles rather than delaying the MFMAs
+                __builtin_amdgcn_s_setprio(1);
+                if (SPLITK && t % 4 == 0) {
+#pragma unroll
+                    for (int r = 0; r < Q; ++r) off[r] = acc{0, 0, 0, 0};
+                    const int ab = (D * nq + min(4 * (t + mfma_reg<T>(j)) + tq, nq - 1)) * NbfP;
+#pragma unroll
+                    for (int s = KF; s < KS; ++s) {
+                        const int k = 4 * s + g, kc = min(k, Nbf - 1);
+                        const bool kin = 4 * s + 3 < Nbf || k < Nbf;
+                        const T av = sT[ab + kc];
+#pragma unroll
+                        for (int r = 0; r < Q; ++r) {
+                            const T b = U[kc + r * Nbf];
+                            off[r] = Mma<T>::mma(av, kin ? b : T(0), off[r]);
+                        }
+                    }
+                }
                 acc C[Q];
 #pragma unroll
                 for (int r = 0; r < Q; ++r) C[r] = acc{0, 0, 0, 0};
                 const int ab = (tc * nq + min(4 * t + tq, nq - 1)) * NbfP;
-                // matrix-core phases run at raised wave priority, so that the SIMD's other wave's
-                // point arithmetic fills the matrix core's busy cycles rather than delaying the MFMAs
-                __builtin_amdgcn_s_setprio(1);
-                {
-                    T av = sT[ab + min(g, Nbf - 1)], b[Q];
 #pragma unroll
-                    for (int r = 0; r < Q; ++r) b[r] = U[min(g, Nbf - 1) + r * Nbf];
+                for (int s = 0; s < KF; ++s) {
+                    const int k = 4 * s + g, kc = min(k, Nbf - 1);
+                    const bool kin = 4 * s + 3 < Nbf || k < Nbf;
+                    const T av = sT[ab + kc];
 #pragma unroll
-                    for (int s = 0; s < KS; ++s) {
-                        const int k = 4 * s + g;
-                        const bool kin = 4 * s + 3 < Nbf || k < Nbf;
-                        T avn = av, bn[Q];
-#pragma unroll
-                        for (int r = 0; r < Q; ++r) bn[r] = b[r];
-                        if (s + 1 < KS) {
-                            const int kn = min(k + 4, Nbf - 1);
-                            avn = sT[ab + kn];
-#pragma unroll
-                            for (int r = 0; r < Q; ++r) bn[r] = U[kn + r * Nbf];
-                        }
-#pragma unroll
-                        for (int r = 0; r < Q; ++r) C[r] = Mma<T>::mma(av, kin ? b[r] : T(0), C[r]);
-                        av = avn;
-#pragma unroll
-                        for (int r = 0; r < Q; ++r) b[r] = bn[r];
+                    for (int r = 0; r < Q; ++r) {
+                        const T b = U[kc + r * Nbf];
+                        C[r] = Mma<T>::mma(av, kin ? b : T(0), C[r]);
                     }
                 }
                 __builtin_amdgcn_s_setprio(0);
+                if constexpr (SPLITK) {
+#pragma unroll
+                    for (int r = 0; r < Q; ++r) {
+                        C[r][D] += off[r][0];
+                        off[r] = acc{off[r][1], off[r][2], off[r][3], 0};
+                    }
+                }
                 // ---- lane (j, g): side sd of facet fl at point q; register c = value (0) / d/dxi_e (1 + e)
                 // rows of G'_s = M_s^-1 with M_s = [t_1 .. t_(D-1), c_s], raw normal t_1 x t_2 (3D)
                 T R[D][D], nr[D], dt;
@@ -367,28 +392,28 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
                         Wt[1 + e][u] = wq * v;
                     }
                 __builtin_amdgcn_s_setprio(1);
-                // ---- lift: Y(k') += sum_(q,c) T0(c, q ; k') W(c, q)
+                // ---- lift: Y(k') += sum_(q,c) T0(c, q ; k') W(c, q); the value and the tangential channels
+                // reach the face's own nodes only (basis tile 0)
                 {
-                    T av = sT[qc * NbfP + min(j, Nbf - 1)];
+                    T av[D + MM];
 #pragma unroll
-                    for (int c = 0; c <= D; ++c) {
+                    for (int c = 0; c < D; ++c) av[c] = sT[(c * nq + qc) * NbfP + min(j, Nbf - 1)];
 #pragma unroll
-                        for (int m = 0; m < MM; ++m) {
-                            const int nx = c * MM + m + 1;
-                            const T avn = nx < (D + 1) * MM
-                                              ? sT[((nx / MM) * nq + qc) * NbfP + min(16 * (nx % MM) + j, Nbf - 1)]
-                                              : av;
+                    for (int m = 0; m < MM; ++m) av[D + m] = sT[(D * nq + qc) * NbfP + min(16 * m + j, Nbf - 1)];
 #pragma unroll
-                            for (int u = 0; u < Q; ++u) Y[m][u] = Mma<T>::mma(av, Wt[c][u], Y[m][u]);
-                            av = avn;
-                        }
-                        if constexpr (VTAIL) {
+                    for (int c = 0; c < D; ++c)
 #pragma unroll
-                            for (int kt = 0; kt < NT; ++kt) {
-                                const T tv = sT[(c * nq + qc) * NbfP + 16 * MM + kt];
+                        for (int u = 0; u < Q; ++u) Y[0][u] = Mma<T>::mma(av[c], Wt[c][u], Y[0][u]);
 #pragma unroll
-                                for (int u = 0; u < Q; ++u) Yt[kt][u] += tv * Wt[c][u];
-                            }
+                    for (int m = 0; m < MM; ++m)
+#pragma unroll
+                        for (int u = 0; u < Q; ++u) Y[m][u] = Mma<T>::mma(av[D + m], Wt[D][u], Y[m][u]);
+                    if constexpr (VTAIL) {
+#pragma unroll
+                        for (int kt = 0; kt < NT; ++kt) {
+                            const T tv = sT[(D * nq + qc) * NbfP + 16 * MM + kt];
+#pragma unroll
+                            for (int u = 0; u < Q; ++u) Yt[kt][u] += tv * Wt[D][u];
                         }
                     }
                 }

@@ -11,6 +11,7 @@ namespace tdg {
 // points:
 //   KS = ceil(Nbf / 4)   K-steps over the basis,         MT = ceil(Nbf / 16) basis tiles,
 //   QB = ceil(Nq / 16)   16-point volume blocks,          FT = ceil(nq / 4)   4-point facet tiles,
+//   KF = ceil(nf / 4)     K-steps over the nf nodes of one face (the first nf labels of the face frame),
 //   NCH = D*D + 2        volume channels (JInv, lamWJ, muWJ),
 //   NFC = 2 D*D + 4 + D  facet channels (own G', lam, mu, neighbour G', lam, mu, oriented normal).
 struct MfmaDims {
@@ -35,6 +36,12 @@ template <int D_, int N_> struct MfmaLayout {
     static constexpr int nq = detail::fct_points(D_, N_);
     static constexpr MfmaDims dims{D_, Nbf, Nq, nq};
     static constexpr int KS = dims.KS, QB = dims.QB, MT = dims.MT, FT = dims.FT, NCH = dims.NCH, NFC = dims.NFC;
+    // Face frame: the basis functions of the nodes off the face vanish on it, so values and tangential
+    // derivatives there involve only the face's own nf nodes (15 of 35 at 3D P4); the normal
+    // derivative involves all.  The face frame numbers the face's nodes first.
+    static constexpr int nf = detail::binom(N_ + D_ - 1, D_ - 1);
+    static constexpr int KF = (nf + 3) / 4;
+    static_assert(nf <= 16, "the face's nodes fit one 16-row tile");
 };
 
 // Output row of a 16x16x4 MFMA tile held in register i (0..3) of lane group g = lane / 16:
@@ -52,8 +59,9 @@ bool mfma_supported(int dim, int degree);
 // element-grouped point data.
 template <class T> struct MfmaArgs {
     T const* V;          // [e][q][k]  d phi_k / d xi_e at volume point q
-    T const* T0;         // [c][q][k]  face-0 value (c = 0) and d/dxi_(c-1) at facet point q
-    int32_t const* perm; // [2][f][k]  facet relabelling perm_f, then its inverse
+    T const* T0;         // [c][q][k]  face-0 value (c = 0) and d/dxi_(c-1) at facet point q, k a face-frame
+                         // label (the face's own nodes first)
+    int32_t const* perm; // [2][f][k]  face-frame label -> element node of face f, then its inverse
     T const* w;          // facet weights
     T const* VD;         // [group][q][NCH][16]
     T const* FD;         // [group][f][q][NFC][16]  both sides' G', lam, mu and the oriented normal
@@ -81,7 +89,7 @@ hipError_t launch_elasticity_mfma(int dim, int degree, MfmaArgs<T> const& a, T c
 template <class T> struct SplitArgs {
     T const* V;
     T const* T0;
-    int32_t const* perm; // [2][f][k] perm_f, then iperm_f
+    int32_t const* perm; // [2][f][k] face-frame label -> element node, then its inverse
     T const* w;
     T const* VD;
     T const* FR;

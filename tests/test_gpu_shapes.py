@@ -1,0 +1,50 @@
+"""Kernel branches at the sizes where they can go wrong, on meshes with permuted vertex ids (every pair
+of local faces meets) against the CPU FP64 oracle.  Bars as in test_gpu_apply.py: relative L2 1e-12 in
+FP64 (observed 1e-14), 1e-5 in FP32 (observed 2e-7)."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import tandem_amd as T
+from cases import BC_D, BC_N, rel_l2, smooth_coefficients, warp_nodes
+
+pytestmark = pytest.mark.gpu
+
+
+class Mixed:
+    """A warped box of n cells with permuted vertex ids, a natural side and Dirichlet elsewhere."""
+
+    def __init__(self, D, n, N, kind=0, seed=0):
+        b = T.Mesh.box(D, n, 1 if D == 3 else 0, [BC_D] * (2 * D - 1) + [BC_N])
+        p = np.random.default_rng(seed).permutation(len(b.vertices))
+        v = np.empty_like(b.vertices)
+        v[p] = b.vertices
+        self.mesh = T.Mesh(v, p[b.elements], p[b.boundary_facets], b.boundary_bc)
+        m = self.mesh
+        self.nodes = np.ascontiguousarray(warp_nodes(m.affine_nodes(N)))
+        self.op = T.DGOperator(m, kind, N, self.nodes)
+        c0, c1 = smooth_coefficients(self.op.volume_points(), seed)
+        self.c = (c0, c1 if kind == 0 else None)
+        self.op.set_material(*self.c)
+        om = O.Mesh.from_arrays(m.vertices, m.elements, m.boundary_facets, m.boundary_bc)
+        self.oracle = O.Operator(kind, om, N, *self.c, nodes=self.nodes)
+        self.n = self.op.n
+
+
+@pytest.mark.parametrize("variant", ["auto", "mfma-element"])
+@pytest.mark.parametrize("D,n,N", [(3, (1, 1, 1), 4), (3, (3, 1, 1), 4), (3, (3, 2, 1), 3), (3, (2, 2, 1), 2),
+                                   (2, (3, 3), 6), (2, (5, 3), 4), (2, (4, 3), 3), (2, (4, 2), 2)])
+def test_face_frame_traces(cuda, D, n, N, variant):
+    """The face frame numbers the face's own nodes first and the facet kernel contracts values and
+    tangential derivatives over those alone: every degree, both sides of its rule, partial groups."""
+    import torch
+
+    c = Mixed(D, n, N, seed=N)
+    c.op.set_variant(variant)
+    x = np.random.default_rng(2).uniform(-1.0, 1.0, c.n)
+    ref = c.oracle.apply(x)
+    for dt, bar in ((torch.float64, 1e-12), (torch.float32, 1e-5)):
+        xd = torch.from_numpy(x).to(cuda).to(dt)
+        y = torch.full_like(xd, float("nan"))
+        c.op.apply(xd, y)
+        assert rel_l2(y.double().cpu().numpy(), ref) <= bar
