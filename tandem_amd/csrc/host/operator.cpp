@@ -942,6 +942,14 @@ RhsArgs Operator::rhs_args() {
             fct[i * 4 + 1] = int32_t(fc.elem[1]);
             fct[i * 4 + 2] = int32_t(fc.local[0]) | (int32_t(fc.local[1]) << 4);
         }
+        std::vector<char> data(E_, 0);
+        for (std::size_t i = 0; i < F; ++i)
+            if (const int bc = fbc[i] & 0xff; bc == BC_Dirichlet || bc == BC_Fault)
+                data[std::size_t(fct[i * 4])] = data[std::size_t(fct[i * 4 + 1])] = 1;
+        std::vector<int32_t> elist;
+        for (std::size_t e = 0; e < E_; ++e)
+            if (data[e]) elist.push_back(int32_t(e));
+        r->elist.upload(elist);
         r->tabE.upload(tabE);
         r->jw.upload(jw);
         r->fbc.upload(fbc);
@@ -964,6 +972,9 @@ RhsArgs Operator::rhs_args() {
     a.ef = reinterpret_cast<int4 const*>(d.ef.ptr);
     a.fbc = rhs64_->fbc.ptr;
     a.fct = reinterpret_cast<int4 const*>(rhs64_->fct.ptr);
+    a.tabFt = d.tabFt.ptr;
+    a.elist = rhs64_->elist.ptr;
+    a.num_elist = int64_t(rhs64_->elist.n);
     a.num_elements = int64_t(E_);
     a.num_facets = int64_t(topo_.facets.size());
     int kq = 0, kf = 0;
@@ -1099,21 +1110,31 @@ WaveArgs Operator::wave_args() {
                 for (unsigned k = 0; k < n; ++k) M[k + l * n] += vol_.weights[q] * E_Q_[k + n * q] * E_Q_[l + n * q];
         for (unsigned k = 0; k < n; ++k) Minv[k + k * n] = 1.0;
         dense_solve(M, int(n), Minv.data(), int(n));
-        std::vector<double> tabE(std::size_t(n) * Nq_), w(E_ * Nq_);
-        for (unsigned k = 0; k < n; ++k)
-            for (unsigned q = 0; q < Nq_; ++q) tabE[k * Nq_ + q] = E_Q_[k + n * q];
-        for (std::size_t e = 0; e < E_; ++e)
-            for (unsigned q = 0; q < Nq_; ++q) w[e * Nq_ + q] = -vol_.weights[q] / absDetJ_[e * Nq_ + q];
+        const bool grouped = inverse_mass_grouped(int(D_), int(N_));
+        std::vector<double> tab(std::size_t(n) * Nq_, 0.0), w(grouped ? (E_ + 15) / 16 * 16 * Nq_ : E_ * Nq_, 0.0);
+        if (grouped) { // P = Mhat^-1 E
+            for (unsigned q = 0; q < Nq_; ++q)
+                for (unsigned l = 0; l < n; ++l)
+                    for (unsigned k = 0; k < n; ++k) tab[q * n + k] += Minv[k + l * n] * E_Q_[l + n * q];
+        } else {
+            for (unsigned k = 0; k < n; ++k)
+                for (unsigned q = 0; q < Nq_; ++q) tab[k * Nq_ + q] = E_Q_[k + n * q];
+        }
+#pragma omp parallel for schedule(static)
+        for (std::size_t e0 = 0; e0 < E_; e0 += 16)
+            for (std::size_t e = e0; e < std::min(e0 + 16, E_); ++e)
+                for (unsigned q = 0; q < Nq_; ++q)
+                    w[grouped ? (e0 * Nq_ + q * 16) + (e - e0) : e * Nq_ + q] =
+                        -vol_.weights[q] / absDetJ_[e * Nq_ + q];
         wv->Minv.upload(Minv);
-        wv->E.upload(tabE);
+        wv->tab.upload(tab);
         wv->w.upload(w);
         wv->ax.alloc(local_size());
-        wv->b.alloc(local_size());
         wave_ = std::move(wv);
     }
     WaveArgs a;
     a.Minv = wave_->Minv.ptr;
-    a.E = wave_->E.ptr;
+    a.E = a.P = wave_->tab.ptr;
     a.w = wave_->w.ptr;
     a.nbf = int(Nbf_);
     a.nq = int(Nq_);
@@ -1124,18 +1145,17 @@ WaveArgs Operator::wave_args() {
 
 void Operator::inverse_mass_device(double const* x, double* y) {
     WaveArgs a = wave_args();
-    TDG_HIP(launch_inverse_mass(a, x, y, stream_));
+    TDG_HIP(launch_inverse_mass(int(D_), int(N_), a, x, y, stream_));
 }
 
 // apply_<true> of Elasticity.cpp:865-880 followed by the inverse mass: y = M^-1 (A x - b_facet(f)).
 void Operator::wave_rhs_device(double const* x, double const* facet_q, double* y) {
     WaveArgs a = wave_args();
     apply(x, wave_->ax.ptr);
-    if (facet_q) {
-        rhs_device(nullptr, facet_q, wave_->b.ptr, 1, 0, 0, 0);
-        TDG_HIP(launch_axpy(wave_->ax.ptr, -1.0, wave_->b.ptr, int64_t(local_size()), stream_));
-    }
-    TDG_HIP(launch_inverse_mass(a, wave_->ax.ptr, y, stream_));
+    if (facet_q)
+        TDG_HIP(launch_elasticity_rhs_facets(int(D_), int(N_), rhs_args(), -1.0, facet_q, wave_->ax.ptr, 1, 0, 0,
+                                             stream_));
+    TDG_HIP(launch_inverse_mass(int(D_), int(N_), a, wave_->ax.ptr, y, stream_));
 }
 
 // I[k][l] = phi^from_l(x^to_k) on the nodal bases (NodalInterpolation.cpp:8-38).

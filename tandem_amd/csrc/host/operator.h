@@ -76,12 +76,13 @@ template <class T> struct DeviceGrad {
 struct DeviceRhs {
     DeviceArray<double> tabE, jw;
     DeviceArray<int32_t> fbc, fct; // fct: int4 per facet
+    DeviceArray<int32_t> elist;    // elements with a Dirichlet or Fault face
 };
 
-// Data of the elastic-wave kernels: reference inverse mass, E table, -W/|J| per volume point and
-// two work vectors.
+// Data of the elastic-wave kernels: reference inverse mass, basis table, -W/|J| per volume point and a
+// work vector.
 struct DeviceWave {
-    DeviceArray<double> Minv, E, w, ax, b;
+    DeviceArray<double> Minv, tab, w, ax; // tab: the basis table E, or P = Mhat^-1 E
 };
 
 // Fault adapter data (FP64) and a work buffer for the facet-point traction of the fault facets.

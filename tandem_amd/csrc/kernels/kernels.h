@@ -53,20 +53,21 @@ template <class T>
 hipError_t launch_material_gradient(int dim, int degree, ApplyArgs<T> const& a, GradArgs<T> const& g, T const* u,
                                     T const* psi, T* g_lam, T* g_mu, hipStream_t stream);
 
-// Weight-adjusted inverse mass (FP64): reference inverse mass, basis at the volume points and the
-// per-point weights -W/|J|.
+// Weight-adjusted inverse mass (FP64): reference inverse mass and basis at the volume points, or their
+// product P = Mhat^-1 E (inverse_mass_grouped operators), and the per-point weights -W/|J|.
 struct WaveArgs {
     double const* Minv; // [Nbf][Nbf] column-major reference inverse mass
     double const* E;    // [k][q] basis at the volume points
-    double const* w;    // [E][Nq] -W / |det J|
+    double const* P;    // [q][k] Mhat^-1 E
+    double const* w;    // -W / |det J|: [E][Nq], or [group of 16 elements][q][16] where grouped
     int nbf, nq, nquant;
     int64_t num_elements;
 };
-hipError_t launch_inverse_mass(WaveArgs const& a, double const* x, double* y, hipStream_t stream);
+bool inverse_mass_grouped(int dim, int degree);
+hipError_t launch_inverse_mass(int dim, int degree, WaveArgs const& a, double const* x, double* y, hipStream_t stream);
 // y = I x per element and quantity (I: n_to x n_from row-major), or y = I^T x if transpose.
 hipError_t launch_interpolate(double const* I, int n_to, int n_from, int nquant, int64_t nelem, int transpose,
                               double const* x, double* y, hipStream_t stream);
-hipError_t launch_axpy(double* y, double alpha, double const* x, int64_t n, hipStream_t stream);
 
 // Assembled block rows (one per element): A[slot][row][col][element] with slot 0 the element's own
 // block and slot 1 + f the block of its face-f neighbour nb[f][element] (the element itself and a zero
@@ -114,9 +115,15 @@ struct RhsArgs {
     int4 const* ef;       // [E][D+1] facet, neighbour, flags
     int32_t const* fbc;   // [F] BC | skeleton << 8
     int4 const* fct;      // [F] element 0, element 1, local face 0 | local face 1 << 4
-    int64_t num_elements, num_facets;
+    double const* tabFt;  // [c][q][k] face-0 facet table, lift order
+    int32_t const* elist; // elements with a Dirichlet or Fault face
+    int64_t num_elements, num_facets, num_elist;
 };
 
+// b(:, c) += sign times the facet part of the rhs for facet data(:, c) (F x Q x nq): only the elements
+// that have a face with data are touched.
+hipError_t launch_elasticity_rhs_facets(int dim, int degree, RhsArgs const& a, double sign, double const* fdata,
+                                        double* b, int ncols, int64_t ld_fdata, int64_t ld_b, hipStream_t stream);
 // b(:, c) = rhs of force(:, c) (E x Q x Nq, may be null) and facet data(:, c) (F x Q x nq, may be
 // null) for ncols columns.
 hipError_t launch_elasticity_rhs(int dim, int degree, RhsArgs const& a, double const* force, double const* fdata,

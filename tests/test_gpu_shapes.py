@@ -48,3 +48,24 @@ def test_face_frame_traces(cuda, D, n, N, variant):
         y = torch.full_like(xd, float("nan"))
         c.op.apply(xd, y)
         assert rel_l2(y.double().cpu().numpy(), ref) <= bar
+
+
+@pytest.mark.parametrize("D,n,N", [(3, (3, 1, 1), 1), (3, (1, 1, 1), 3), (2, (3, 3), 1), (2, (3, 5), 2), (2, (4, 2), 4),
+                                   (2, (9, 1), 5), (3, (1, 1, 1), 5)])
+def test_wave_rhs_degrees(cuda, D, n, N):
+    """The matrix-core inverse mass at the other degrees and partial groups (3D P5 keeps the kernel with
+    run-time sizes and has no apply), in place too; the facet part added to the elements with data."""
+    import torch
+
+    c = Mixed(D, n, N, seed=N)
+    rng = np.random.default_rng(4)
+    x, g = rng.uniform(-1.0, 1.0, c.n), rng.uniform(-1.0, 1.0, (c.op.F, D, c.op.nq))
+    xd, gd = torch.from_numpy(x).to(cuda), torch.from_numpy(g.ravel()).to(cuda)
+    assert rel_l2(c.op.inverse_mass(xd).cpu().numpy(), c.oracle.inverse_mass(x)) <= 1e-12
+    z = xd.clone()
+    assert rel_l2(c.op.inverse_mass(z, z).cpu().numpy(), c.oracle.inverse_mass(x)) <= 1e-12
+    if D == 3 and N > 4:
+        return
+    assert rel_l2(c.op.wave_rhs(xd, gd).cpu().numpy(), c.oracle.wave_rhs(x, g)) <= 1e-12
+    b = torch.empty_like(xd)
+    assert rel_l2(c.op.rhs_device(b, None, gd).cpu().numpy(), c.oracle.rhs(None, g)) <= 1e-12
