@@ -558,9 +558,15 @@ std::vector<double> Operator::autotune_shapes(int ncols, int pb) {
     if (!(kind_ == Kind_Elasticity && mfma_supported(D_, N_)))
         return std::vector<double>(kSplitOrders * kSplitShapes, -1.0);
     const int saved_variant = variant_, saved_shape = split_shape_[p], saved_xcd = split_xcd_[p];
+    const bool saved_auto = split_auto_[p];
+    // the last configuration: the automatic choice, which takes the small applies' shape
+    const int last = kSplitOrders * kSplitShapes;
+    const bool small = split_is_small(pb, ncols);
     try {
         variant_ = Variant_Auto;
-        time_configs(ncols, pb, kSplitOrders * kSplitShapes, [&](int c) {
+        time_configs(ncols, pb, last + 1, [&](int c) {
+            split_auto_[p] = c == last;
+            if (c == last) return small;
             split_shape_[p] = c / kSplitOrders;
             split_xcd_[p] = c % kSplitOrders;
             return true;
@@ -569,14 +575,17 @@ std::vector<double> Operator::autotune_shapes(int ncols, int pb) {
         variant_ = saved_variant;
         split_shape_[p] = saved_shape;
         split_xcd_[p] = saved_xcd;
+        split_auto_[p] = saved_auto;
         throw;
     }
     variant_ = saved_variant;
     int best = 0;
-    for (int c = 1; c < kSplitOrders * kSplitShapes; ++c)
+    for (int c = 1; c < last; ++c)
         if (ms[std::size_t(c)] >= 0.0 && ms[std::size_t(c)] < ms[std::size_t(best)]) best = c;
     split_shape_[p] = best / kSplitOrders;
     split_xcd_[p] = best % kSplitOrders;
+    split_auto_[p] = small && ms[std::size_t(last)] < ms[std::size_t(best)];
+    ms.resize(std::size_t(last));
     return ms;
 }
 
@@ -614,6 +623,19 @@ void Operator::set_split_shape(int pb, int shape, int xcd) {
         throw std::invalid_argument("bad launch shape");
     split_shape_[pb == 8 ? 0 : 1] = shape;
     split_xcd_[pb == 8 ? 0 : 1] = xcd;
+    split_auto_[pb == 8 ? 0 : 1] = false;
+}
+
+// Launch shape and workgroup order the two-kernel apply of ncols columns runs with.
+void Operator::split_choice(int pb, int ncols, int& shape, int& order) const {
+    const int p = pb == 8 ? 0 : 1;
+    const bool small = split_auto_[p] && split_is_small(pb, ncols);
+    shape = small ? kSplitSmall : split_shape_[p];
+    order = small ? 0 : split_xcd_[p];
+}
+
+bool Operator::split_is_small(int pb, int ncols) const {
+    return int64_t((E_ + 15) / 16) * ncols <= split_small_groups(pb);
 }
 
 bool Operator::uses_mfma() const {
@@ -1577,11 +1599,11 @@ template <class T> void Operator::dispatch(T const* x, T* y, int ncols, int64_t 
         }();
         reserve_split(ds, ncols);
         const int64_t ldL = int64_t(E_) * (D_ + 1) * int64_t(block_size());
-        const int p = sizeof(T) == 8 ? 0 : 1;
         SplitArgs<T> sa = split_args(dm, ds);
-        sa.xcd_remap = split_xcd_[p];
-        TDG_HIP(launch_elasticity_split<T>(D_, N_, split_shape_[p], sa, x, y, ds.L.ptr, ncols, ncols > 1 ? ld : 0,
-                                           ldL, stream_));
+        int shape = 0;
+        split_choice(int(sizeof(T)), ncols, shape, sa.xcd_remap);
+        TDG_HIP(launch_elasticity_split<T>(D_, N_, shape, sa, x, y, ds.L.ptr, ncols, ncols > 1 ? ld : 0, ldL,
+                                           stream_));
     } else if (uses_mfma()) {
         if constexpr (std::is_same<T, double>::value) launch_mfma(*m64_, x, y, ncols, ld);
         else launch_mfma(*m32_, x, y, ncols, ld);
@@ -1596,7 +1618,7 @@ int64_t Operator::dot_partials_capacity() const {
     if (!(kind_ == Kind_Elasticity && mfma_supported(D_, N_))) return 0;
     const int64_t ng = int64_t((E_ + 15) / 16);
     int64_t m = 0;
-    for (int sh = 0; sh < kSplitShapes; ++sh)
+    for (int sh = 0; sh <= kSplitSmall; ++sh)
         m = std::max({m, split_element_workgroups<double>(sh, ng), split_element_workgroups<float>(sh, ng)});
     return m;
 }
@@ -1619,13 +1641,13 @@ template <class T> int64_t Operator::apply_dot_impl(T const* x, T* y, double* pa
         if constexpr (std::is_same<T, double>::value) return *m64_;
         else return *m32_;
     }();
-    const int p = sizeof(T) == 8 ? 0 : 1;
     SplitArgs<T> sa = split_args(dm, ds);
-    sa.xcd_remap = split_xcd_[p];
+    int shape = 0;
+    split_choice(int(sizeof(T)), 1, shape, sa.xcd_remap);
     sa.dot = partials;
     const int64_t ldL = int64_t(E_) * (D_ + 1) * int64_t(block_size());
-    TDG_HIP(launch_elasticity_split<T>(D_, N_, split_shape_[p], sa, x, y, ds.L.ptr, 1, 0, ldL, stream_));
-    return split_element_workgroups<T>(split_shape_[p], int64_t((E_ + 15) / 16));
+    TDG_HIP(launch_elasticity_split<T>(D_, N_, shape, sa, x, y, ds.L.ptr, 1, 0, ldL, stream_));
+    return split_element_workgroups<T>(shape, int64_t((E_ + 15) / 16));
 }
 
 int64_t Operator::apply_dot(double const* x, double* y, double* partials) { return apply_dot_impl(x, y, partials); }
@@ -1662,8 +1684,9 @@ void Operator::apply_noalloc(double const* x, double* y, double* scratch, std::s
         throw std::runtime_error("no kernel compiled for this dimension/degree");
     TDG_HIP(launch_zero_slots<double>(scratch, s64_->idle.ptr, int64_t(s64_->idle.n), int(block_size()), stream_));
     SplitArgs<double> sa = split_args(*m64_, *s64_);
-    sa.xcd_remap = split_xcd_[0];
-    TDG_HIP(launch_elasticity_split<double>(D_, N_, split_shape_[0], sa, x, y, scratch, 1, 0, int64_t(need), stream_));
+    int shape = 0;
+    split_choice(8, 1, shape, sa.xcd_remap);
+    TDG_HIP(launch_elasticity_split<double>(D_, N_, shape, sa, x, y, scratch, 1, 0, int64_t(need), stream_));
 }
 void Operator::apply(float const* x, float* y) { dispatch(x, y, 1, 0); }
 void Operator::apply_batched(double const* X, double* Y, int ncols, int64_t ld) { dispatch(X, Y, ncols, ld); }

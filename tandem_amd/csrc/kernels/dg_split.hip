@@ -19,7 +19,7 @@ TDG_SPLIT_DECL(2, 6)
 template <class T>
 hipError_t launch_elasticity_split(int dim, int degree, int shape, SplitArgs<T> const& a, T const* x, T* y, T* L,
                                    int ncols, int64_t ld, int64_t ldL, hipStream_t s) {
-    if (shape < 0 || shape >= kSplitShapes) return hipErrorInvalidValue;
+    if (shape < 0 || shape > kSplitSmall) return hipErrorInvalidValue;
     if (dim == 3) {
         switch (degree) {
         case 2: return launch_split_d3p2<T>(shape, a, x, y, L, ncols, ld, ldL, s);

@@ -114,7 +114,9 @@ __device__ __forceinline__ double mirror16(double v) {
     return __builtin_bit_cast(double, (static_cast<unsigned long long>(unsigned(hi)) << 32) | unsigned(lo));
 }
 
-template <int D, int N, class T, int W, int OCC, bool VTAIL_ON, bool PERSIST>
+// SPL > 1 (small meshes): SPL consecutive waves share 8 facets, each taking every SPL-th tile, and sum
+// their lifted rows in LDS.
+template <int D, int N, class T, int W, int OCC, bool VTAIL_ON, bool PERSIST, int SPL = 1>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(OCC)))
 void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __restrict__ Ls, int64_t ld,
                              int64_t ldL, int ncols, unsigned nvb) {
@@ -126,7 +128,8 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
     // derivative only) four tiles at a time, where that spares at least 5 K-steps a wave (3D P4: 5 x 9
     // -> 5 x 4 + 2 x 5, P3: 4 x 5 -> 4 x 3 + 2, 2D P6: 2 x 7 -> 2 x 2 + 5).  With fewer the extra pass
     // costs more than it spares (3D P2, 2 x 3 -> 2 x 2 + 1: 28.2 -> 29.3 us at 14,586 elements, FP64).
-    constexpr bool SPLITK = (FT - (FT + 3) / 4) * (KS - L::KF) >= 5;
+    static_assert(W % SPL == 0 && (SPL == 1 || (SPL <= FT && !PERSIST)), "whole groups of waves");
+    constexpr bool SPLITK = SPL == 1 && (FT - (FT + 3) / 4) * (KS - L::KF) >= 5;
     constexpr int KF = SPLITK ? L::KF : KS;
     constexpr int NFR = DD + D + 4; // tangents (D-1 columns), c_0, c_1, lam_0, mu_0, lam_1, mu_1
     constexpr int NbfP = Strides<T>::pad(Nbf), BSP = Strides<T>::pad(BS);
@@ -166,7 +169,8 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
         T* const X = sX[wv];
         unsigned col, lb;
         block_of(vb, nvb, ncols, a.xcd_remap, col, lb);
-        const int64_t grp = int64_t(lb) * W + wv;
+        const int part = SPL > 1 ? wv % SPL : 0;
+        const int64_t grp = int64_t(lb) * (W / SPL) + wv / SPL;
         const bool live = grp < a.num_fgroups; // uniform per wave
         const int64_t gj = live ? grp : 0;
         T const* __restrict__ x = xs + int64_t(col) * ld;
@@ -193,7 +197,7 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
             rc[DD + 1] = r[(chl + 1) * 8];
         };
         T rc[DD + 2];
-        load_rec(0, rc);
+        load_rec(part, rc);
 
         // element vector of this column in LDS, relabelled to face 0: U'(k', r) = x(perm_f(k'), r);
         // lane (j, g) moves entries 4 i + g
@@ -234,12 +238,12 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
             acc off[Q];
 
 #pragma unroll 1
-            for (int t = 0; t < FT; ++t) {
+            for (int t = part; t < FT; t += SPL) {
                 const int q = 4 * t + g;
                 const int qc = min(q, nq - 1);
                 const bool act = ok && q < nq;
                 T rn[DD + 2];
-                load_rec(min(t + 1, FT - 1), rn); // next tile's record, one tile ahead
+                load_rec(min(t + SPL, FT - 1), rn); // next tile's record, one tile ahead
                 // quadrature weight, zero on lanes without a facet point (every lane computes finite
                 // values: padding facets carry the identity Jacobian, empty columns a zero vector)
                 const T wq = act ? sW[qc] : T(0);
@@ -460,12 +464,20 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
                 }
             }
         }
-        wave_sync();
+        if constexpr (SPL == 1) wave_sync();
+        else __syncthreads();
         if (ok) {
             T* const dst = Lc + (int64_t(el) * NF + lf) * BS + g;
 #pragma unroll
-            for (int i = 0; i < NI; ++i)
-                if (4 * i + 3 < BS || 4 * i + g < BS) dst[4 * i] = X[j * BSP + 4 * i + g];
+            for (int ii = 0; ii < (NI + SPL - 1) / SPL; ++ii) {
+                const int i = SPL * ii + part;
+                if (4 * i + 3 < BS || 4 * i + g < BS) {
+                    T v = sX[wv - part][j * BSP + 4 * i + g];
+#pragma unroll
+                    for (int s = 1; s < SPL; ++s) v += sX[wv - part + s][j * BSP + 4 * i + g];
+                    dst[4 * i] = v;
+                }
+            }
         }
         wave_sync(); // every read of the staged region is done before the next block restages it
     };
@@ -481,7 +493,9 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
 // block b and the facet slots during the last block, so only the first loads of a wave wait on
 // memory.  Otherwise (two or more waves per SIMD) each block loads its own point data up front and
 // the slots are read at the end; the other waves of the SIMD cover the waits.
-template <int D, int N, class T, int W, int OCC, bool DEEP, bool VTAIL_ON, bool PERSIST>
+// SPL > 1 (small meshes): SPL consecutive waves share 16 elements, each taking every SPL-th block of
+// points, and sum their results from LDS as they store them.
+template <int D, int N, class T, int W, int OCC, bool DEEP, bool VTAIL_ON, bool PERSIST, int SPL = 1>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(OCC)))
 void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const* __restrict__ Ls,
                                T* __restrict__ ys, int64_t ld, int64_t ldL, int ncols, unsigned nvb) {
@@ -495,7 +509,9 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
     constexpr bool VTAIL = VTAIL_ON && D == 3 && MT > 1 && TAIL <= 4;
     constexpr int MM = VTAIL ? MT - 1 : MT;
     constexpr int NT = VTAIL ? TAIL : 1;
-    constexpr int NO = (16 * BS + 63) / 64; // output entries per lane
+    constexpr int NX = (16 * BS + 63) / 64;      // staged entries per lane
+    constexpr int NO = (NX + SPL - 1) / SPL;     // output entries per lane: 64 (SPL o + part) + lane
+    static_assert(W % SPL == 0 && (SPL == 1 || (SPL <= QB && !PERSIST && !DEEP)), "whole groups of waves");
 
     __shared__ T sV[D * Nq * NbfP];
     __shared__ T sU[W][16 * BSP];
@@ -513,7 +529,8 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         T* const U = sU[wv];
         unsigned col, lb;
         block_of(vb, nvb, ncols, a.xcd_remap, col, lb);
-        const int64_t grp = int64_t(lb) * W + wv;
+        const int part = SPL > 1 ? wv % SPL : 0;
+        const int64_t grp = int64_t(lb) * (W / SPL) + wv / SPL;
         const bool live = grp < a.num_groups; // uniform per wave
         T const* __restrict__ x = xs + int64_t(col) * ld;
         T const* __restrict__ Lc = Ls + int64_t(col) * ldL;
@@ -540,7 +557,7 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         auto load_slots = [&](T (&ls)[NO]) {
 #pragma unroll
             for (int o = 0; o < NO; ++o) {
-                const int i = 64 * o + lane;
+                const int i = 64 * (SPL * o + part) + lane;
                 const int ic = min(i, max(nout - 1, 0));
                 const int jj = ic / BS, rem = ic - jj * BS;
                 T v = T(0);
@@ -554,11 +571,11 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         if constexpr (DEEP) load_pd(0, pd);
         if (live) {
             // every load first (clamped addresses), then the LDS stores: no load waits on another
-            T v[NO];
+            T v[NX];
 #pragma unroll
-            for (int o = 0; o < NO; ++o) v[o] = xw[min(64 * o + lane, nout - 1)];
+            for (int o = 0; o < NX; ++o) v[o] = xw[min(64 * o + lane, nout - 1)];
 #pragma unroll
-            for (int o = 0; o < NO; ++o) {
+            for (int o = 0; o < NX; ++o) {
                 const int i = 64 * o + lane;
                 if (i < 16 * BS) U[(i / BS) * BSP + i % BS] = i < nout ? v[o] : T(0);
             }
@@ -683,7 +700,7 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
                 }
             } else {
 #pragma unroll 1
-                for (int b = 0; b < QB; ++b) {
+                for (int b = part; b < QB; b += SPL) {
                     // the point data are loaded before the matrix-core work that does not need them:
                     // FP32 all four registers; FP64 (fewer registers to spare) two, and the other two
                     // once the block's reference-gradient MFMAs are issued
@@ -732,19 +749,23 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         T xv[NO];
         if (a.dot && live) {
 #pragma unroll
-            for (int o = 0; o < NO; ++o) xv[o] = xw[min(64 * o + lane, nout - 1)];
+            for (int o = 0; o < NO; ++o) xv[o] = xw[min(64 * (SPL * o + part) + lane, nout - 1)];
         }
-        wave_sync();
+        if constexpr (SPL == 1) wave_sync();
+        else __syncthreads();
         double dot = 0.0;
         if (live) {
             // y = volume + the element's facet slots
             T* dst = y + e0 * BS;
 #pragma unroll
             for (int o = 0; o < NO; ++o) {
-                const int i = 64 * o + lane;
+                const int i = 64 * (SPL * o + part) + lane;
                 if (i < nout) {
                     const int jj = i / BS, rem = i - jj * BS;
-                    const T v = U[jj * BSP + rem] + ls[o];
+                    T v = sU[wv - part][jj * BSP + rem];
+#pragma unroll
+                    for (int s = 1; s < SPL; ++s) v += sU[wv - part + s][jj * BSP + rem];
+                    v += ls[o];
                     dst[i] = v;
                     if (a.dot) dot += double(xv[o]) * double(v);
                 }
@@ -831,10 +852,36 @@ hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols
     return hipGetLastError();
 }
 
+// Small meshes: G groups of 16 elements (8 facets) per workgroup, each shared by as many waves as it has
+// blocks of points (tiles).  A mesh of a few hundred groups otherwise occupies a few CUs with waves that
+// each run one long chain of matrix-core steps.  The results do not depend on G.
+template <int D, int N, class T, int G>
+hipError_t run_small(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
+                     hipStream_t s) {
+    using L = MfmaLayout<D, N>;
+    const int64_t ft = ((a.num_fgroups + G - 1) / G + 7) / 8 * 8 * int64_t(ncols);
+    const int64_t et = ((a.num_groups + G - 1) / G + 7) / 8 * 8 * int64_t(ncols);
+    if (ft > int64_t(0x7fffffff) || et > int64_t(0x7fffffff)) return hipErrorInvalidValue;
+    if (ft > 0) {
+        hipLaunchKernelGGL((elasticity_facet_kernel<D, N, T, G * L::FT, 2, true, false, L::FT>), dim3(unsigned(ft)),
+                           dim3(64 * G * L::FT), 0, s, a, x, Lbuf, ld, ldL, ncols, unsigned(ft));
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((elasticity_element_kernel<D, N, T, G * L::QB, 2, false, true, false, L::QB>),
+                       dim3(unsigned(et)), dim3(64 * G * L::QB), 0, s, a, x, Lbuf, y, ld, ldL, ncols, unsigned(et));
+    return hipGetLastError();
+}
+inline int64_t small_workgroups(int64_t num_groups) { return (num_groups + 7) / 8 * 8; } // one column: G = 1
+
 // The shape table (index < kSplitShapes): FP64 kernels hold up to two waves per SIMD, FP32 more.
 template <int D, int N, class T>
 hipError_t run_split(int shape, SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
                      hipStream_t s) {
+    if (shape == kSplitSmall)
+        // two groups a workgroup share the tables once every CU has work
+        return a.num_groups * ncols <= kSmallOneGroup ? run_small<D, N, T, 1>(a, x, y, Lbuf, ncols, ld, ldL, s)
+                                                      : run_small<D, N, T, 2>(a, x, y, Lbuf, ncols, ld, ldL, s);
     if constexpr (sizeof(T) == 8) {
         switch (shape) {
         case 0: return run_shape<D, N, T, Shape<4, 2, 8, 2, false, true>>(a, x, y, Lbuf, ncols, ld, ldL, s);
@@ -854,6 +901,8 @@ hipError_t run_split(int shape, SplitArgs<T> const& a, T const* x, T* y, T* Lbuf
 }
 
 template <class T> int64_t element_workgroups_of(int shape, int64_t num_groups) {
+    if (shape == kSplitSmall)
+        return num_groups <= kSmallOneGroup ? small_workgroups(num_groups) : small_workgroups((num_groups + 1) / 2);
     if constexpr (sizeof(T) == 8) {
         switch (shape) {
         case 0: return element_workgroups<Shape<4, 2, 8, 2, false, true>>(num_groups);

@@ -104,6 +104,17 @@ template <class T> struct SplitArgs {
 // Number of launch shapes of the two-kernel apply (waves per workgroup, occupancy targets, element
 // prefetch depth, lift tail on the vector ALU or the matrix cores), per precision.
 constexpr int kSplitShapes = 4;
+// Launch shape of small applies: the waves of a workgroup share each group of elements (facets), one
+// group a workgroup up to kSmallOneGroup groups x columns, then two.  Taken up to split_small_groups
+// groups of 16 elements x columns.  us per apply, other shapes -> this one, at 24 / 192 / 375 / 648 groups:
+//   3D P4 FP64  70 -> 24, 75 -> 54, 84 -> 73, 94 -> 116     FP32  35 -> 18, 37 -> 36, 45 -> 53, 50 -> 80
+//   3D P3 FP64  35 -> 16, 38 -> 29, 45 -> 38, 53 -> 54      FP32  19 -> 13, 20 -> 18, 25 -> 26, 31 -> 34
+//   3D P2 FP64  18 -> 12, 19 -> 15,  -      , 26 -> 27      FP32  11 -> 10, 12 -> 12,  -      , 15 -> 19
+// (2D P6 and P4 alike; 16 columns of 24 groups: P4 FP64 86 -> 75, FP32 47 -> 53).  Above, the other shapes
+// win: two waves a SIMD share one table and nothing is summed across waves.
+constexpr int kSplitSmall = kSplitShapes;
+constexpr int64_t kSmallOneGroup = 256;
+constexpr int64_t split_small_groups(int precision_bytes) { return precision_bytes == 8 ? 384 : 192; }
 // Workgroup orders (SplitArgs::xcd_remap) searched with each shape.
 constexpr int kSplitOrders = 3;
 

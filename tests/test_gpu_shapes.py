@@ -69,3 +69,44 @@ def test_wave_rhs_degrees(cuda, D, n, N):
     assert rel_l2(c.op.wave_rhs(xd, gd).cpu().numpy(), c.oracle.wave_rhs(x, g)) <= 1e-12
     b = torch.empty_like(xd)
     assert rel_l2(c.op.rhs_device(b, None, gd).cpu().numpy(), c.oracle.rhs(None, g)) <= 1e-12
+
+
+@pytest.mark.parametrize("D,n,N", [(3, (1, 1, 1), 4), (3, (3, 2, 1), 4), (3, (3, 2, 1), 3), (3, (2, 2, 1), 2),
+                                   (2, (3, 3), 6), (2, (5, 3), 4), (2, (3, 3), 3)])
+def test_small_apply_and_explicit_shapes(cuda, D, n, N):
+    """The shape of small applies (default here), with the fused dot product of the solvers, and every
+    explicitly chosen launch shape and workgroup order on the same mesh."""
+    import torch
+
+    c = Mixed(D, n, N, seed=N + 1)
+    x = np.random.default_rng(3).uniform(-1.0, 1.0, c.n)
+    ref = c.oracle.apply(x)
+    for prec, dt, bar in (("fp64", torch.float64, 1e-12), ("fp32", torch.float32, 1e-5)):
+        xd = torch.from_numpy(x).to(cuda).to(dt)
+        for config in [None] + [(s, o) for s in range(4) for o in range(3)]:
+            if config:
+                c.op.set_shape(prec, *config)
+            y = torch.full_like(xd, float("nan"))
+            c.op.apply(xd, y)
+            assert rel_l2(y.double().cpu().numpy(), ref) <= bar, config
+
+
+@pytest.mark.parametrize("D,n,N,cols", [(3, (4, 4, 4), 4, 17), (2, (16, 16), 6, 25), (3, (8, 7, 7), 2, 1)])
+def test_small_apply_limits(cuda, D, n, N, cols):
+    """Groups x columns on both sides of the rule (384 FP64, 192 FP32 groups of 16 elements) and of the
+    one-group-a-workgroup limit, batched and singly; a short CG runs the fused dot on the small shape."""
+    import torch
+
+    c = Mixed(D, n, N, seed=5)
+    X = np.random.default_rng(6).uniform(-1.0, 1.0, (cols, c.n))
+    ref = np.stack([c.oracle.apply(x, nthreads=4) for x in X])
+    for dt, bar in ((torch.float64, 1e-12), (torch.float32, 1e-5)):
+        for k in sorted({1, min(cols, 7), min(cols, 11), cols - 1 or 1, cols}):
+            Xd = torch.from_numpy(X[:k]).to(cuda).to(dt)
+            Y = torch.full_like(Xd, float("nan"))
+            c.op.apply_batched(Xd, Y)
+            assert rel_l2(Y.double().cpu().numpy(), ref[:k]) <= bar, k
+    b = torch.from_numpy(ref[0]).to(cuda)
+    x = torch.zeros_like(b)
+    res = c.op.solve(b, x, rtol=1e-8, mode="fp64", precond="block-jacobi", max_iter=5000)
+    assert res["converged"] and rel_l2(c.oracle.apply(x.cpu().numpy()), ref[0]) <= 1e-7
