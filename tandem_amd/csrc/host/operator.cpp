@@ -405,6 +405,8 @@ void Operator::drop_device() {
     m32_.reset();
     s64_.reset();
     s32_.reset();
+    p64_.reset();
+    p32_.reset();
     rhs64_.reset();
     bj_.reset();
     asm_.reset();
@@ -452,6 +454,8 @@ void Operator::upload_device() {
     } else if (uses_mfma()) {
         ensure_mfma_faces();
     }
+    if (uses_poisson_mfma(8, 1)) device_poisson<double>();
+    if (uses_poisson_mfma(4, 1)) device_poisson<float>();
     if (variant_ == Variant_Assembled && !asm_) assemble(); // before any graph capture of the apply
 }
 
@@ -477,6 +481,8 @@ void Operator::reserve_columns(int ncols) {
         reserve_split(*s64_, ncols);
         reserve_split(*s32_, ncols);
     }
+    if (uses_poisson_mfma(8, ncols)) reserve_poisson(device_poisson<double>(), ncols);
+    if (uses_poisson_mfma(4, ncols)) reserve_poisson(device_poisson<float>(), ncols);
 }
 
 template <class T> void Operator::reserve_split(DeviceSplit<T>& ds, int ncols) {
@@ -603,7 +609,10 @@ std::vector<double> Operator::autotune(int ncols, int pb) {
                 variant_ = v;
                 return true;
             }
-            if (v != Variant_Points && !mfma) return false;
+            if (v != Variant_Points && !mfma) {
+                variant_ = v;
+                return v == Variant_Auto && uses_poisson_mfma(pb, ncols);
+            }
             variant_ = v;
             return true;
         }, ms);
@@ -825,6 +834,110 @@ template <class T> void Operator::upload_split(DeviceSplit<T>& ds) {
     ds.ntwo = int64_t(ntwo);
     ds.cap = 0;
     reserve_split(ds, 1);
+}
+
+bool Operator::uses_poisson_mfma(int pb, int ncols) const {
+    int kq = 0, kf = 0;
+    return kind_ == Kind_Poisson && variant_ == Variant_Auto && kernel_rule_sizes(D_, N_, &kq, &kf) == 0 &&
+           kq == int(Nq_) && kf == int(nq_) && !(D_ == 2 && N_ == 1) &&
+           int64_t(local_size()) * ncols >= poisson_mfma_unknowns(int(D_), pb);
+}
+
+template <class T> DevicePoisson<T>& Operator::device_poisson() {
+    auto& slot = [&]() -> auto& {
+        if constexpr (std::is_same<T, double>::value) return p64_;
+        else return p32_;
+    }();
+    if (!slot) {
+        auto d = std::make_unique<DevicePoisson<T>>();
+        upload_poisson(*d);
+        slot = std::move(d);
+    }
+    return *slot;
+}
+
+template <class T> void Operator::reserve_poisson(DevicePoisson<T>& d, int ncols) {
+    if (d.cap >= ncols) return;
+    d.TR.alloc(trace_entries() * std::size_t(ncols));
+    d.cap = ncols;
+}
+
+// Point data of the matrix-core Poisson apply in groups of 16 elements, element innermost (layouts and
+// meaning at PoissonArgs).
+template <class T> void Operator::upload_poisson(DevicePoisson<T>& d) {
+    const unsigned D = D_, DD = D * D, NF = D + 1, C = D + 1, NS = D * (D + 1) / 2;
+    std::vector<double> V(std::size_t(D) * Nq_ * Nbf_), F(std::size_t(NF) * C * nq_ * Nbf_);
+    for (unsigned e = 0; e < D; ++e)
+        for (unsigned q = 0; q < Nq_; ++q)
+            for (unsigned k = 0; k < Nbf_; ++k) V[(e * Nq_ + q) * Nbf_ + k] = Dxi_Q_[k + Nbf_ * (e + D * q)];
+    for (unsigned f = 0; f < NF; ++f)
+        for (unsigned c = 0; c < C; ++c)
+            for (unsigned q = 0; q < nq_; ++q)
+                for (unsigned k = 0; k < Nbf_; ++k)
+                    F[((f * C + c) * nq_ + q) * Nbf_ + k] =
+                        c == 0 ? E_q_[f][k + Nbf_ * q] : Dxi_q_[f][k + Nbf_ * ((c - 1) + D * q)];
+    const std::size_t ng = (E_ + 15) / 16;
+    std::vector<T> PV(ng * Nq_ * NS * 16, T(0)), PK(ng * NF * nq_ * C * 16, T(0));
+    std::vector<int32_t> PF(ng * NF * 16 * 2, 0);
+#pragma omp parallel for schedule(static)
+    for (std::size_t e = 0; e < E_; ++e) {
+        const std::size_t grp = e / 16, j = e % 16;
+        for (unsigned q = 0; q < Nq_; ++q) {
+            double const* G = &JInv_[(e * Nq_ + q) * DD];
+            T* o = &PV[(grp * Nq_ + q) * NS * 16 + j];
+            for (unsigned a = 0, c = 0; a < D; ++a)
+                for (unsigned b = a; b < D; ++b, ++c) {
+                    double v = 0.0;
+                    for (unsigned r = 0; r < D; ++r) v += G[a + r * D] * G[b + r * D];
+                    o[c * 16] = T(c0Q_[e * Nq_ + q] * v);
+                }
+        }
+        for (unsigned f = 0; f < NF; ++f) {
+            int32_t const* ef = &ef_[(e * NF + f) * 4];
+            const std::size_t fct = std::size_t(ef[0]);
+            const int side = (ef[2] >> 2) & 1;
+            int32_t* pf = &PF[((grp * NF + f) * 16 + j) * 2];
+            pf[0] = ef[1];
+            pf[1] = ((ef[2] >> 4) & 3) | ((ef[2] & 3) << 4);
+            for (unsigned q = 0; q < nq_; ++q) {
+                double const* K = &fGp_[((fct * 2 + side) * nq_ + q) * DD];
+                double const* n = &normal_[(fct * nq_ + q) * D];
+                T* o = &PK[((grp * NF + f) * nq_ + q) * C * 16 + j];
+                for (unsigned a = 0; a < D; ++a) {
+                    double v = 0.0;
+                    for (unsigned r = 0; r < D; ++r) v += K[a + r * D] * n[r];
+                    o[a * 16] = T(side ? -v : v);
+                }
+                o[D * 16] = T(penalty_[fct] * nlen_[fct * nq_ + q]);
+            }
+        }
+    }
+    d.V.upload(cast<T>(V));
+    d.F.upload(cast<T>(F));
+    d.w.upload(cast<T>(fct_.weights));
+    d.PV.upload(PV);
+    d.PK.upload(PK);
+    d.PF.upload(PF);
+    d.cap = 0;
+    reserve_poisson(d, 1);
+}
+
+template <class T> void Operator::launch_poisson_device(T const* x, T* y, T* TR, int ncols, int64_t ld) {
+    DevicePoisson<T>& d = device_poisson<T>();
+    if (!TR) {
+        reserve_poisson(d, ncols);
+        TR = d.TR.ptr;
+    }
+    PoissonArgs<T> a;
+    a.V = d.V.ptr;
+    a.F = d.F.ptr;
+    a.w = d.w.ptr;
+    a.PV = d.PV.ptr;
+    a.PK = d.PK.ptr;
+    a.PF = reinterpret_cast<int2 const*>(d.PF.ptr);
+    a.num_elements = int64_t(E_);
+    TDG_HIP(launch_poisson_mfma<T>(int(D_), int(N_), a, x, y, TR, ncols, ncols > 1 ? ld : 0,
+                                   int64_t(trace_entries()), stream_));
 }
 
 template <class T> static std::vector<T> cast(std::vector<double> const& v) {
@@ -1607,6 +1720,8 @@ template <class T> void Operator::dispatch(T const* x, T* y, int ncols, int64_t 
     } else if (uses_mfma()) {
         if constexpr (std::is_same<T, double>::value) launch_mfma(*m64_, x, y, ncols, ld);
         else launch_mfma(*m32_, x, y, ncols, ld);
+    } else if (uses_poisson_mfma(int(sizeof(T)), ncols)) {
+        launch_poisson_device<T>(x, y, nullptr, ncols, ld);
     } else {
         launch(device<T>(), x, y, ncols, ld);
     }
@@ -1670,6 +1785,13 @@ void Operator::apply_noalloc(double const* x, double* y, double* scratch, std::s
     if (!have)
         throw std::logic_error("the allocation-free apply needs the operator on the device: call tdg_upload "
                                "(or one tdg_mult) first");
+    if (uses_poisson_mfma(8, 1)) {
+        // the traces go to the scratch memory; operators whose traces it cannot hold, or that were uploaded for
+        // another variant, take the kernel without any
+        if (p64_ && trace_entries() <= cap) launch_poisson_device<double>(x, y, scratch, 1, 0);
+        else launch(*d64_, x, y, 1, 0);
+        return;
+    }
     if (!uses_split()) { // the other kernels use no scratch memory
         dispatch(x, y, 1, 0);
         return;

@@ -46,6 +46,7 @@ template <class T> struct DeviceOperator {
 
 template <class T> struct MfmaArgs;
 template <class T> struct SplitArgs;
+template <class T> struct PoissonArgs;
 
 // Operand tables and element-grouped point data of the MFMA elasticity kernel (one precision).
 template <class T> struct DeviceMfma {
@@ -63,6 +64,14 @@ template <class T> struct DeviceSplit {
     DeviceArray<int32_t> idle;  // slots (element * (D+1) + face) of faces without a facet term
     DeviceArray<T> L;
     int64_t nfacets = 0, ntwo = 0;
+    int cap = 0;
+};
+
+// Tables and element-grouped point data of the matrix-core Poisson apply (PoissonArgs), and the traces
+// of its two kernels (cap columns).
+template <class T> struct DevicePoisson {
+    DeviceArray<T> V, F, w, PV, PK, TR;
+    DeviceArray<int32_t> PF; // int2 per element face
     int cap = 0;
 };
 
@@ -263,6 +272,13 @@ private:
     template <class T> void upload_split(DeviceSplit<T>& d);
     template <class T> SplitArgs<T> split_args(DeviceMfma<T> const& m, DeviceSplit<T> const& s) const;
     template <class T> void reserve_split(DeviceSplit<T>& s, int ncols);
+    // whether an apply of ncols columns in pb bytes a real takes the matrix-core Poisson kernels
+    bool uses_poisson_mfma(int pb, int ncols) const;
+    template <class T> DevicePoisson<T>& device_poisson();
+    template <class T> void upload_poisson(DevicePoisson<T>& d);
+    template <class T> void reserve_poisson(DevicePoisson<T>& d, int ncols);
+    template <class T> void launch_poisson_device(T const* x, T* y, T* TR, int ncols, int64_t ld);
+    std::size_t trace_entries() const { return E_ * (D_ + 1) * nq_ * 2; }
     template <class T> int64_t apply_dot_impl(T const* x, T* y, double* partials);
     void ensure_mfma_faces();
     template <class T> void launch(DeviceOperator<T> const& d, T const* x, T* y, int ncols, int64_t ld);
@@ -309,6 +325,8 @@ private:
     std::unique_ptr<DeviceMfma<float>> m32_;
     std::unique_ptr<DeviceSplit<double>> s64_;
     std::unique_ptr<DeviceSplit<float>> s32_;
+    std::unique_ptr<DevicePoisson<double>> p64_;
+    std::unique_ptr<DevicePoisson<float>> p32_;
     std::unique_ptr<DeviceRhs> rhs64_;
     std::unique_ptr<BlockJacobi> bj_;
     std::unique_ptr<DeviceAssembled> asm_;

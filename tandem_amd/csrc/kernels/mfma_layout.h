@@ -131,6 +131,36 @@ template <class T> int64_t split_element_workgroups(int shape, int64_t num_group
 // Zeroes the facet slots listed in `slots` (slot s = entries [s bs, (s + 1) bs) of L).
 template <class T> hipError_t launch_zero_slots(T* L, int32_t const* slots, int64_t nslots, int bs, hipStream_t s);
 
+// Arguments of the two-kernel matrix-core Poisson apply (element-grouped data, element innermost):
+//   V  [e][q][k]                    modal basis gradients at the volume points
+//   F  [f][c][q][k]                 face f's values (c = 0) and gradients at its points
+//   PV [group][q][D (D + 1) / 2][16]  upper triangle of W|J| K G G^T by rows
+//   PK [group][f][q][D + 1][16]     K G n (n outward, area-scaled), then penalty |n|
+//   PF [group][f][16]               {neighbour, its face | kind << 4}
+template <class T> struct PoissonArgs {
+    T const* V;
+    T const* F;
+    T const* w;
+    T const* PV;
+    T const* PK;
+    int2 const* PF;
+    int64_t num_elements;
+};
+// y = A x for ncols columns (stride ld) through the traces TR[element][f][q] = {u, K grad u . n} (column
+// stride ldT = E (D + 1) nq 2).
+template <class T>
+hipError_t launch_poisson_mfma(int dim, int degree, PoissonArgs<T> const& a, T const* x, T* y, T* TR, int ncols,
+                               int64_t ld, int64_t ldT, hipStream_t stream);
+// Unknowns x columns from which the matrix-core Poisson apply is taken.  us per apply, thread-per-point
+// kernel -> this one (two launches and their tables cost 8 us in 2D, 10 to 45 in 3D whatever the size):
+//   FP64  2D P2   49k 7.0 -> 8.6  120k 13.4 -> 10.6   P4  31k 6.9 -> 11.6  123k 18 -> 12   P6  57k 17 -> 17
+//         3D P1   12k 7.8 -> 8.9   41k 12.9 -> 9.6    P2  31k 13.2 -> 13.3  104k 34 -> 15   P4  45k 61 -> 46
+//   FP32  2D P3   82k 6.4 -> 8.5  120k (P2) 10.7 -> 9.5   3D P4  45k 33 -> 39  108k 48 -> 39
+// 2D P1 stays with the thread-per-point kernel: 540k unknowns 32 -> 28 in FP64, 20 -> 23 in FP32.
+constexpr int64_t poisson_mfma_unknowns(int dim, int precision_bytes) {
+    return dim == 2 ? (precision_bytes == 8 ? 70000 : 120000) : (precision_bytes == 8 ? 32000 : 64000);
+}
+
 template <class T> struct GradArgs;
 // Adjoint material gradient on the matrix cores (same dimensions and degrees as the apply):
 // g_lam, g_mu (E x Nq) = d/d(lam_Q, mu_Q) of psi^T A u.

@@ -110,3 +110,38 @@ def test_small_apply_limits(cuda, D, n, N, cols):
     x = torch.zeros_like(b)
     res = c.op.solve(b, x, rtol=1e-8, mode="fp64", precond="block-jacobi", max_iter=5000)
     assert res["converged"] and rel_l2(c.oracle.apply(x.cpu().numpy()), ref[0]) <= 1e-7
+
+
+@pytest.mark.parametrize("D,n,N", [(2, (101, 101), 2), (2, (79, 77), 3), (2, (65, 63), 4), (2, (55, 53), 5),
+                                   (2, (47, 47), 6), (3, (15, 13, 14), 1), (3, (11, 10, 10), 2), (3, (9, 9, 7), 3),
+                                   (3, (7, 7, 7), 4)])
+def test_poisson_matrix_core_apply(cuda, D, n, N):
+    """Every compiled degree of the matrix-core Poisson apply (both kernels, natural and Dirichlet faces,
+    a partial last group) just above its size rule, singly, batched at a larger stride, without
+    allocation; "points" agrees."""
+    import ctypes as C
+
+    import torch
+    from tandem_amd._lib import lib
+
+    c = Mixed(D, n, N, kind=1, seed=N)
+    assert c.op.E % 16 != 0
+    X = np.random.default_rng(8).uniform(-1.0, 1.0, (3, c.n))
+    ref = np.stack([c.oracle.apply(x, nthreads=4) for x in X])
+    for dt, bar in ((torch.float64, 1e-12), (torch.float32, 1e-5)):
+        Xd = torch.zeros((3, c.n + 6), dtype=dt, device=cuda)
+        Xd[:, :c.n] = torch.from_numpy(X).to(cuda).to(dt)
+        Y = torch.full_like(Xd, float("nan"))
+        c.op.apply_batched(Xd, Y)
+        assert rel_l2(Y[:, :c.n].double().cpu().numpy(), ref) <= bar
+        y = torch.full((c.n,), float("nan"), dtype=dt, device=cuda)
+        c.op.apply(Xd[1, :c.n].contiguous(), y)
+        assert torch.equal(y, Y[1, :c.n])
+        if dt == torch.float64:
+            z = torch.full_like(y, float("nan"))
+            assert lib().tdg_mult_noalloc(c.op._h, C.c_void_p(Xd[1].contiguous().data_ptr()), C.c_void_p(z.data_ptr())) == 0
+            assert torch.equal(z, y)
+        c.op.set_variant("points")
+        c.op.apply(Xd[1, :c.n].contiguous(), y)
+        assert rel_l2(y.double().cpu().numpy(), ref[1]) <= bar
+        c.op.set_variant("auto")
