@@ -1550,6 +1550,8 @@ template <class T> AssembledArgs<T> Operator::assembled_args() const {
     a.slots = int(D_ + 2);
     return a;
 }
+template AssembledArgs<double> Operator::assembled_args<double>() const;
+template AssembledArgs<float> Operator::assembled_args<float>() const;
 
 void Operator::traction_device(double const* x, double const* facet_q, double* t) {
     if (!ready_) throw std::logic_error("set_material() must be called first");

@@ -231,6 +231,8 @@ public:
     // Host copies of the FP64 block rows (A[slot][row][col][element]) and face neighbours
     // (nb[face][element]); assembles first if needed.
     void assembled_host(std::vector<double>& A, std::vector<int32_t>& nb);
+    // Device view of the assembled block rows (assembled before).
+    template <class T> AssembledArgs<T> assembled_args() const;
     SimplexMesh const& mesh() const { return mesh_; }
 
     // g_lam, g_mu (E x Nq, device) = d/d(lam_Q, mu_Q) of psi^T A u for device vectors u, psi
@@ -285,7 +287,6 @@ private:
     template <class T> MfmaArgs<T> mfma_args(DeviceMfma<T> const& d) const;
     template <class T> void launch_mfma(DeviceMfma<T> const& d, T const* x, T* y, int ncols, int64_t ld);
     template <class T> void dispatch(T const* x, T* y, int ncols, int64_t ld);
-    template <class T> AssembledArgs<T> assembled_args() const;
     template <class T> bool apply_batched_dot_impl(T const* X, T* Y, int ncols, int64_t ld, double* partial);
 
     int kind_;

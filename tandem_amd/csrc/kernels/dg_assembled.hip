@@ -16,11 +16,15 @@
 //     block) and writing R entries of y.  The matrix is read from HBM once per
 //     column range instead of once per column, so a 64-column apply costs little more than the
 //     64 x / y column reads and writes.
+//   * row kernel (the register kernel's block sizes, at most kFewColumns columns): a lane per element row,
+//     32 elements of all rows a workgroup, so that a coarse level of a few thousand elements fills the chip
+//     for one column, and the multigrid smoother's block-Jacobi and Chebyshev update ride on the product.
 //   * generic kernel (any block size; the cross-check of the matrix-free apply at high order): one
 //     lane per element row and column, the block row streamed from HBM per column.
 #include "kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace tdg {
 
@@ -133,6 +137,66 @@ __global__ __launch_bounds__(kThreads) void assembled_apply_kernel(AssembledArgs
     }
 }
 
+// Row kernel: lane (element, row), 32 consecutive elements fastest (every block-row load of a half wave
+// is one contiguous 32-element piece), columns in grid.y; sums in the register kernel's order.  With one
+// element per lane, 3,072 elements of 12 rows were 48 waves of 720 multiply-adds each: 15.6 us a product,
+// and 27 us a smoothing step in four launches.
+enum RowMode { Row_Apply, Row_Residual, Row_Smooth };
+constexpr int kRowElements = 32;
+template <class T, int BS, int NB, int MODE>
+__global__ __launch_bounds__(kRowElements* BS) void assembled_row_kernel(AssembledArgs<T> a, AssembledStep<T> p) {
+    __shared__ T sR[BS][kRowElements];
+    const int l = threadIdx.x % kRowElements, row = threadIdx.x / kRowElements;
+    const int64_t E = a.num_elements, e = int64_t(blockIdx.x) * kRowElements + l, c = blockIdx.y;
+    const bool act = e < E;
+    const int64_t ec = act ? e : E - 1, i = ec * BS + row;
+    T acc = T(0);
+    T const* const x = p.x ? p.x + c * p.ldx : nullptr;
+    if (MODE != Row_Smooth || x) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int64_t off = (b == 0 ? ec : int64_t(a.nb[int64_t(b - 1) * E + ec])) * BS;
+#pragma unroll
+            for (int j = 0; j < BS; ++j) acc += a.A[((int64_t(b) * BS + row) * BS + j) * E + ec] * x[off + j];
+        }
+    }
+    T* const out = p.out + c * p.ldo;
+    if constexpr (MODE == Row_Apply) {
+        if (act) out[i] = acc;
+    } else if constexpr (MODE == Row_Residual) {
+        if (act) out[i] = p.b[c * p.ldb + i] - acc;
+    } else {
+        sR[row][l] = p.b[c * p.ldb + i] - acc;
+        __syncthreads();
+        T z = T(0);
+#pragma unroll
+        for (int j = 0; j < BS; ++j) z += p.Dinv[ec * (BS * BS) + row + j * BS] * sR[j][l];
+        if (!act) return;
+        T* const d = p.d + c * p.ldd + i;
+        const T dv = p.c1 != T(0) ? p.c1 * *d + p.c2 * z : p.c2 * z;
+        *d = dv;
+        out[i] = x ? x[i] + dv : dv;
+    }
+}
+
+template <int MODE, class T>
+hipError_t run_rows(AssembledArgs<T> const& a, AssembledStep<T> const& p, int ncols, hipStream_t s) {
+    const int64_t gx = (a.num_elements + kRowElements - 1) / kRowElements;
+    if (gx > int64_t(0x7fffffff)) return hipErrorInvalidValue;
+    const dim3 g{unsigned(gx), unsigned(ncols)};
+    const int bs = a.block_size;
+    auto run = [&](auto Bs, auto Nb) {
+        constexpr int B = decltype(Bs)::value, NB = decltype(Nb)::value;
+        hipLaunchKernelGGL((assembled_row_kernel<T, B, NB, MODE>), g, dim3(kRowElements * B), 0, s, a, p);
+        return hipGetLastError();
+    };
+    using std::integral_constant;
+    if (a.slots == 4 && bs == 6) return run(integral_constant<int, 6>{}, integral_constant<int, 4>{});
+    if (a.slots == 4 && bs == 12) return run(integral_constant<int, 12>{}, integral_constant<int, 4>{});
+    if (a.slots == 5 && bs == 12) return run(integral_constant<int, 12>{}, integral_constant<int, 5>{});
+    return hipErrorNotSupported;
+}
+
 // One lane per (row, element), element fastest (coalesced block-row reads), one column per grid row.
 template <class T>
 __global__ __launch_bounds__(kThreads) void assembled_apply_generic(AssembledArgs<T> a, T const* __restrict__ xs,
@@ -209,6 +273,14 @@ hipError_t launch_assembled(AssembledArgs<T> const& a, T const* x, T* y, int nco
     if (ncols > 1 && ld < a.num_elements * a.block_size) return hipErrorInvalidValue;
     if (ncols > 65535 * kDotCols) return hipErrorInvalidValue;
     const int bs = a.block_size;
+    if (!partial && ncols <= kFewColumns) {
+        AssembledStep<T> p;
+        p.x = x;
+        p.out = y;
+        p.ldx = p.ldo = ncols > 1 ? ld : 0;
+        const hipError_t e = run_rows<Row_Apply>(a, p, ncols, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     if (a.slots == 4) {
         if (bs == 3) return run_bs<T, 3, 4>(a, x, y, ncols, ld, partial, s);
         if (bs == 6) return run_bs<T, 6, 4>(a, x, y, ncols, ld, partial, s);
@@ -224,6 +296,22 @@ hipError_t launch_assembled(AssembledArgs<T> const& a, T const* x, T* y, int nco
     return hipGetLastError();
 }
 
+template <class T>
+hipError_t launch_assembled_residual(AssembledArgs<T> const& a, AssembledStep<T> const& p, int ncols, hipStream_t s) {
+    return run_rows<Row_Residual>(a, p, ncols, s);
+}
+template <class T>
+hipError_t launch_assembled_smooth(AssembledArgs<T> const& a, AssembledStep<T> const& p, int ncols, hipStream_t s) {
+    return run_rows<Row_Smooth>(a, p, ncols, s);
+}
+template hipError_t launch_assembled_residual<float>(AssembledArgs<float> const&, AssembledStep<float> const&, int,
+                                                     hipStream_t);
+template hipError_t launch_assembled_residual<double>(AssembledArgs<double> const&, AssembledStep<double> const&, int,
+                                                      hipStream_t);
+template hipError_t launch_assembled_smooth<float>(AssembledArgs<float> const&, AssembledStep<float> const&, int,
+                                                   hipStream_t);
+template hipError_t launch_assembled_smooth<double>(AssembledArgs<double> const&, AssembledStep<double> const&, int,
+                                                    hipStream_t);
 template hipError_t launch_assembled<double>(AssembledArgs<double> const&, double const*, double*, int, int64_t,
                                              hipStream_t, double*);
 template hipError_t launch_assembled<float>(AssembledArgs<float> const&, float const*, float*, int, int64_t,

@@ -88,6 +88,25 @@ template <class T>
 hipError_t launch_assembled(AssembledArgs<T> const& a, T const* x, T* y, int ncols, int64_t ld, hipStream_t stream,
                             double* partial = nullptr);
 bool assembled_register_kernel(int block_size, int slots);
+// Few columns (ncols <= kFewColumns): the row kernel (a lane per element row) with a fused epilogue.
+//   Residual  out = b - A x
+//   Smooth    z = Dinv (b - A x), d = c1 d + c2 z, out = x + d; x null: the zero guess (out must not be x)
+// Vectors at strides ld (x, out, d) and ldb (b); Dinv[element][bs x bs] column-major.  Block sizes 6 and 12
+// with 4 slots, 12 with 5; hipErrorNotSupported otherwise.
+constexpr int kFewColumns = 2;
+template <class T> struct AssembledStep {
+    T const* b = nullptr;
+    T const* x = nullptr;
+    T* out = nullptr;
+    T* d = nullptr;
+    T const* Dinv = nullptr;
+    int64_t ldb = 0, ldx = 0, ldo = 0, ldd = 0;
+    T c1 = 0, c2 = 0;
+};
+template <class T>
+hipError_t launch_assembled_residual(AssembledArgs<T> const& a, AssembledStep<T> const& p, int ncols, hipStream_t s);
+template <class T>
+hipError_t launch_assembled_smooth(AssembledArgs<T> const& a, AssembledStep<T> const& p, int ncols, hipStream_t s);
 // Assembly by probing (FP64): X (m columns of E bs) = unit vectors c0 .. c0 + m - 1 on the elements of
 // colour c; gather stores the isolated block columns of Y = A X into the assembled layout.
 hipError_t launch_assembly_probe(double* X, int32_t const* colour, int c, int c0, int m, int64_t E, int bs,

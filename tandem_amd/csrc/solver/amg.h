@@ -58,6 +58,8 @@ private:
     template <class T> void run(T const* r, T* z, int ncols, int64_t ld);
     template <class T> void smooth(int l, T const* b, int64_t ldb, T* x, int64_t ldx, int ncols, bool zero_guess);
     template <class T>
+    void step(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* out, int64_t ldo, int ncols, int k);
+    template <class T>
     void residual(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* r, int64_t ldr, int ncols);
     template <class T> void cycle(int l, T const* b, int64_t ldb, T* x, int64_t ldx, int ncols);
 

@@ -3,6 +3,7 @@
 #include "amg.h"
 
 #include "../host/operator.h"
+#include "../kernels/kernels.h"
 #include "../host/refelem.h"
 #include "block_jacobi.h"
 #include "multi_kernels.h"
@@ -355,17 +356,81 @@ __global__ __launch_bounds__(kT) void bsr_kernel(int64_t n, int64_t const* __res
     }
 }
 
-// x = Ainv b (dense N x N, row-major), ncols columns
+// Few columns: one wave per block row, its lanes (slice, row r of the blocks): slice s takes every
+// SL-th block, the slices' sums meet in shuffles.  A level of a few hundred block rows is latency bound:
+// with a lane per scalar row each walked its 20 to 40 blocks alone (10 us a product at 600 block rows).
+// MODE 3, one Chebyshev step: z = Dinv (b - A x), d = c1 d + c2 z, y = x + d (x null: the zero guess).
+template <class T> struct BsrStep {
+    T const* Dinv = nullptr;
+    T* d = nullptr;
+    int64_t ldd = 0;
+    T c1 = 0, c2 = 0;
+};
+template <class T, int BR, int BC, int MODE>
+__global__ __launch_bounds__(kT) void bsr_wave_kernel(int64_t n, int64_t const* __restrict__ rp,
+                                                      int32_t const* __restrict__ ci, T const* __restrict__ v,
+                                                      T const* xs, int64_t ldx, T* ys, int64_t ldy,
+                                                      T const* __restrict__ bs, int64_t ldb, BsrStep<T> p) {
+    constexpr int SL = 64 / BR; // slices of the block row's blocks
+    const int64_t i = int64_t(blockIdx.x) * (kT / 64) + threadIdx.x / 64;
+    if (i >= n) return; // whole waves
+    const int lane = threadIdx.x & 63, sl = lane / BR, r = lane - sl * BR;
+    const int64_t c = blockIdx.y;
+    T acc = T(0);
+    if (sl < SL && (MODE != 3 || xs)) {
+        T const* x = xs + c * ldx;
+        for (int64_t k = rp[i] + sl; k < rp[i + 1]; k += SL) {
+            T const* b = v + k * (BR * BC) + r * BC;
+            T const* xv = x + int64_t(ci[k]) * BC;
+#pragma unroll
+            for (int s = 0; s < BC; ++s) acc += b[s] * xv[s];
+        }
+    }
+    // pairwise over the slices (the lanes past the last slice hold zero)
+    constexpr int P2 = SL > 16 ? 32 : SL > 8 ? 16 : SL > 4 ? 8 : 4;
+#pragma unroll
+    for (int h = P2 / 2; h > 0; h /= 2) {
+        const T o = __shfl_down(acc, unsigned(h * BR), 64);
+        if (sl < h && sl + h < SL) acc += o;
+    }
+    const int64_t t = i * BR + r;
+    T* const y = ys + c * ldy + t;
+    if constexpr (MODE == 3) {
+        const T res = sl == 0 ? bs[c * ldb + t] - acc : T(0);
+        T z = T(0);
+#pragma unroll
+        for (int s = 0; s < BR; ++s) {
+            const T rs = __shfl(res, s, 64);
+            if (sl == 0) z += p.Dinv[t * BR + s] * rs;
+        }
+        if (sl != 0) return;
+        T* const d = p.d + c * p.ldd + t;
+        const T dv = p.c1 != T(0) ? p.c1 * *d + p.c2 * z : p.c2 * z;
+        *d = dv;
+        *y = xs ? xs[c * ldx + t] + dv : dv;
+    } else {
+        if (sl != 0) return;
+        if constexpr (MODE == 0) *y = acc;
+        else if constexpr (MODE == 1) *y = bs[c * ldb + t] - acc;
+        else *y += acc;
+    }
+}
+
+// x = Ainv b (dense N x N, row-major), ncols columns: one wave per row (a lane per row left the
+// at most 800 rows on 13 waves that walked a row each: 27 us)
 template <class T>
 __global__ __launch_bounds__(kT) void dense_kernel(int64_t N, T const* __restrict__ Ainv, T const* __restrict__ bs,
                                                    int64_t ldb, T* __restrict__ xs, int64_t ldx) {
-    const int64_t i = int64_t(blockIdx.x) * kT + threadIdx.x;
-    if (i >= N) return;
+    const int64_t i = int64_t(blockIdx.x) * (kT / 64) + threadIdx.x / 64;
+    if (i >= N) return; // whole waves
+    const int lane = threadIdx.x & 63;
     T const* b = bs + int64_t(blockIdx.y) * ldb;
     T const* a = Ainv + i * N;
     T s = T(0);
-    for (int64_t j = 0; j < N; ++j) s += a[j] * b[j];
-    xs[int64_t(blockIdx.y) * ldx + i] = s;
+    for (int64_t j = lane; j < N; j += 64) s += a[j] * b[j];
+#pragma unroll
+    for (int o = 32; o > 0; o /= 2) s += __shfl_down(s, unsigned(o), 64);
+    if (lane == 0) xs[int64_t(blockIdx.y) * ldx + i] = s;
 }
 
 // d = z / theta; x = d (zero guess) or x += d
@@ -459,10 +524,17 @@ struct DevBsr {
 template <int MODE, class T>
 void bsr_launch(DevBsr const& A, T const* x, int64_t ldx, T* y, int64_t ldy, T const* b, int64_t ldb, int ncols,
                 hipStream_t s) {
-    const dim3 g(blocks_for(A.n * A.br), unsigned(ncols)), t(kT);
+    const bool few = ncols <= kFewColumns;
+    const dim3 g(few ? unsigned((A.n + kT / 64 - 1) / (kT / 64)) : blocks_for(A.n * A.br), unsigned(ncols)), t(kT);
     T const* v = A.values<T>();
 #define TDG_BSR(R, C)                                                                                        \
     if (A.br == R && A.bc == C) {                                                                            \
+        if (few) {                                                                                           \
+            hipLaunchKernelGGL((bsr_wave_kernel<T, R, C, MODE>), g, t, 0, s, A.n, A.rp.p, A.ci.p, v, x, ldx,   \
+                               y, ldy, b, ldb, BsrStep<T>{});                                                \
+            MHIP(hipGetLastError());                                                                         \
+            return;                                                                                          \
+        }                                                                                                    \
         hipLaunchKernelGGL((bsr_kernel<T, R, C, MODE>), g, t, 0, s, A.n, A.rp.p, A.ci.p, v, x, ldx, y, ldy, b,   \
                            ldb);                                                                             \
         MHIP(hipGetLastError());                                                                             \
@@ -478,6 +550,20 @@ void bsr_launch(DevBsr const& A, T const* x, int64_t ldx, T* y, int64_t ldy, T c
     TDG_BSR(6, 12)
 #undef TDG_BSR
     throw std::logic_error("AMG: no kernel for this block shape");
+}
+
+// One Chebyshev step (few columns) on a square operator with 3 x 3 or 6 x 6 blocks.
+template <class T>
+void bsr_smooth(DevBsr const& A, T const* x, int64_t ldx, T* y, int64_t ldy, T const* b, int64_t ldb,
+                BsrStep<T> const& p, int ncols, hipStream_t s) {
+    const dim3 g(unsigned((A.n + kT / 64 - 1) / (kT / 64)), unsigned(ncols)), t(kT);
+    if (A.br == 3)
+        hipLaunchKernelGGL((bsr_wave_kernel<T, 3, 3, 3>), g, t, 0, s, A.n, A.rp.p, A.ci.p, A.values<T>(), x, ldx, y,
+                           ldy, b, ldb, p);
+    else
+        hipLaunchKernelGGL((bsr_wave_kernel<T, 6, 6, 3>), g, t, 0, s, A.n, A.rp.p, A.ci.p, A.values<T>(), x, ldx, y,
+                           ldy, b, ldb, p);
+    MHIP(hipGetLastError());
 }
 
 // Work vectors of one level in one precision.
@@ -650,12 +736,60 @@ AMG::AMG(Operator& op, AMGOptions const& o) : op_(op), o_(o) {
 
 AMG::~AMG() = default;
 
+// Chebyshev step k of a smoothing from x (null: the zero guess) to out, few columns.
+template <class T>
+void AMG::step(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* out, int64_t ldo, int ncols, int k) {
+    AMGLevelDev& v = *lv_[l];
+    LevelVectors<T>& w = v.w<T>();
+    const double lo = o_.eig_lo * rho_[l], hi = o_.eig_hi * rho_[l];
+    const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
+    double c1 = 0.0, c2 = 1.0 / theta, rho0 = 1.0 / sigma;
+    for (int j = 1; j <= k; ++j) {
+        const double rho1 = 1.0 / (2.0 * sigma - rho0);
+        c1 = rho1 * rho0;
+        c2 = 2.0 * rho1 / delta;
+        rho0 = rho1;
+    }
+    if (l == 0) {
+        AssembledStep<T> p;
+        p.b = b;
+        p.x = x;
+        p.out = out;
+        p.d = w.d.p;
+        p.Dinv = op_.block_jacobi().blocks<T>();
+        p.ldb = ldb;
+        p.ldx = ldx;
+        p.ldo = ldo;
+        p.ldd = v.ld;
+        p.c1 = T(c1);
+        p.c2 = T(c2);
+        MHIP(launch_assembled_smooth<T>(op_.assembled_args<T>(), p, ncols, op_.stream()));
+    } else {
+        BsrStep<T> p;
+        p.Dinv = v.Dinv.values<T>();
+        p.d = w.d.p;
+        p.ldd = v.ld;
+        p.c1 = T(c1);
+        p.c2 = T(c2);
+        bsr_smooth<T>(v.A, x, ldx, out, ldo, b, ldb, p, ncols, op_.stream());
+    }
+}
+
 // r = b - A_l x
 template <class T>
 void AMG::residual(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* r, int64_t ldr, int ncols) {
     AMGLevelDev& v = *lv_[l];
     hipStream_t st = op_.stream();
-    if (l == 0) {
+    if (l == 0 && ncols <= kFewColumns) {
+        AssembledStep<T> p;
+        p.b = b;
+        p.x = x;
+        p.out = r;
+        p.ldb = ldb;
+        p.ldx = ldx;
+        p.ldo = ldr;
+        MHIP(launch_assembled_residual<T>(op_.assembled_args<T>(), p, ncols, st));
+    } else if (l == 0) {
         T* t = v.w<T>().t.p;
         op_.apply_batched(x, t, ncols, v.ld);
         const int64_t N = v.n * v.bs;
@@ -707,14 +841,35 @@ template <class T> void AMG::cycle(int l, T const* b, int64_t ldb, T* x, int64_t
     hipStream_t st = op_.stream();
     if (l + 1 == int(lv_.size())) {
         const int64_t N = v.n * v.bs;
-        hipLaunchKernelGGL((dense_kernel<T>), dim3(blocks_for(N), unsigned(ncols)), dim3(kT), 0, st, N, v.dense<T>(), b,
-                           ldb, x, ldx);
+        hipLaunchKernelGGL((dense_kernel<T>), dim3(unsigned((N + kT / 64 - 1) / (kT / 64)), unsigned(ncols)), dim3(kT),
+                           0, st, N, v.dense<T>(), b, ldb, x, ldx);
         MHIP(hipGetLastError());
         return;
     }
     AMGLevelDev& c = *lv_[l + 1];
     LevelVectors<T>& w = v.w<T>();
     LevelVectors<T>& wc = c.w<T>();
+    if (ncols <= kFewColumns) {
+        // every step is one launch that reads the neighbours' old x and writes the other vector
+        T *u[2] = {w.z.p, w.t.p}, *cur = nullptr;
+        for (int k = 0; k < o_.smooth; ++k) {
+            step<T>(l, b, ldb, cur, v.ld, u[k & 1], v.ld, ncols, k);
+            cur = u[k & 1];
+        }
+        residual<T>(l, b, ldb, cur, v.ld, w.r.p, v.ld, ncols);
+        bsr_launch<0>(v.R, static_cast<T const*>(w.r.p), v.ld, wc.b.p, c.ld, static_cast<T const*>(nullptr), 0, ncols,
+                      st);
+        cycle<T>(l + 1, wc.b.p, c.ld, wc.x.p, c.ld, ncols);
+        bsr_launch<2>(v.P, static_cast<T const*>(wc.x.p), c.ld, cur, v.ld, static_cast<T const*>(nullptr), 0, ncols,
+                      st);
+        for (int k = 0; k < o_.smooth; ++k) {
+            const bool last = k + 1 == o_.smooth;
+            T* const out = last ? x : cur == u[0] ? u[1] : u[0];
+            step<T>(l, b, ldb, cur, v.ld, out, last ? ldx : v.ld, ncols, k);
+            cur = out;
+        }
+        return;
+    }
     smooth<T>(l, b, ldb, x, ldx, ncols, true);
     residual<T>(l, b, ldb, x, ldx, w.r.p, v.ld, ncols);
     bsr_launch<0>(v.R, static_cast<T const*>(w.r.p), v.ld, wc.b.p, c.ld, static_cast<T const*>(nullptr), 0, ncols, st);
@@ -740,7 +895,7 @@ template <class T> void AMG::run(T const* r, T* z, int ncols, int64_t ld) {
                 w.r.ensure(tot);
                 w.d.ensure(tot);
                 w.z.ensure(tot);
-                if (l == 0) w.t.ensure(tot);
+                w.t.ensure(tot);
             }
         }
         cap_cols_[p] = ncols;

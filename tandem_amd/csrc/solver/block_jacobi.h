@@ -48,6 +48,11 @@ public:
     bool apply_dot(double const* r, double* z, hipStream_t s, int ncols, int64_t ld, double* partial,
                    bool fp32_blocks) const;
 
+    // Whole inverse blocks on the device ([element][bs x bs] column-major; null where they are packed).
+    template <class T> T const* blocks() const {
+        if constexpr (sizeof(T) == 8) return inv64_;
+        else return inv32_;
+    }
     // FP64 inverse block of element e (bs x bs, column-major) copied to the host, for checks.
     void inverse_block(int64_t e, double* out) const;
 

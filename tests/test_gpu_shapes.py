@@ -145,3 +145,36 @@ def test_poisson_matrix_core_apply(cuda, D, n, N):
         c.op.apply(Xd[1, :c.n].contiguous(), y)
         assert rel_l2(y.double().cpu().numpy(), ref[1]) <= bar
         c.op.set_variant("auto")
+
+
+@pytest.mark.parametrize("fp32", [1, 0])
+@pytest.mark.parametrize("D,n,degrees", [(3, (4, 3, 5), (2, 1)), (2, (15, 13), (2, 1)), (2, (15, 13), (3, 2))])
+def test_multigrid_few_columns(cuda, D, n, degrees, fp32):
+    """The coarse solver's kernels for at most two columns (assembled rows of 6 and 12, fused smoothing
+    steps, a wave per block row) and, with three columns, those for many: the same solutions to 1e-10."""
+    import torch
+
+    cs = [Mixed(D, n, N, seed=9) for N in degrees]
+    fine, ops = cs[0], [c.op for c in cs]
+    assert ops[-1].n > 800 and ops[-1].E % 32 != 0
+    B = np.random.default_rng(12).uniform(-1.0, 1.0, (3, fine.n))
+    Bd = torch.zeros((3, fine.n + 4), dtype=torch.float64, device=cuda)
+    Bd[:, :fine.n] = torch.from_numpy(B).to(cuda)
+    mg = T.PMultigrid(ops, galerkin_penalty=0, vcycle_fp32=fp32, coarse_fp32=fp32)
+    for k in (1, 2, 3):
+        X = torch.zeros((k, fine.n + 4), dtype=torch.float64, device=cuda)
+        res = mg.solve_multi(Bd[:k].contiguous(), X, rtol=1e-10)
+        assert res["converged"]
+        for c in range(k):
+            r = B[c] - fine.oracle.apply(X[c, :fine.n].cpu().numpy())
+            assert np.linalg.norm(r) <= 1e-9 * np.linalg.norm(B[c])
+    op = ops[-1]  # assembled by the set-up: two columns at a stride equal single applies
+    for dt in (torch.float64, torch.float32):
+        X = torch.rand((2, op.n + 3), dtype=dt, device=cuda)
+        Y = torch.full_like(X, 7.0)
+        op.apply_batched(X, Y)
+        for c in range(2):
+            y = torch.zeros(op.n, dtype=dt, device=cuda)
+            op.apply(X[c, :op.n].contiguous(), y)
+            assert torch.equal(y, Y[c, :op.n])
+        assert torch.all(Y[:, op.n:] == 7.0)
