@@ -144,9 +144,9 @@ int tdg_autotune(tdg_op* op, int ncols, int precision_bytes, int* chosen, double
  * on ncols columns in FP64 (precision_bytes 8) or FP32 (4), keeps the fastest for that precision,
  * reports it in *shape and *xcd and the milliseconds per apply in ms[TDG_SPLIT_ORDERS shape + xcd]
  * (TDG_SPLIT_ORDERS x TDG_SPLIT_SHAPES entries, -1 if the operator has no two-kernel apply).  tdg_set_shape selects one directly.
- * Until a shape is selected, applies of few elements (384 groups of 16 elements times columns in FP64,
- * 192 in FP32) run with a shape made for them, whose workgroups share each group; the search keeps that
- * choice for such operators where it is the faster one.  tdg_autotune runs the shape search before it compares the variants.  No counterpart in the reference (its kernels are
+ * Until a shape is selected, applies of few elements (up to 1024 groups of 16 elements times columns, or
+ * 384 groups of 8 facets) run with launches made for them, whose waves share each group; the search keeps
+ * those for such operators where they are the faster choice.  tdg_autotune runs the shape search before it compares the variants.  No counterpart in the reference (its kernels are
  * generated for one CPU target). */
 enum { TDG_SPLIT_SHAPES = 4, TDG_SPLIT_ORDERS = 3 };
 int tdg_autotune_shapes(tdg_op* op, int ncols, int precision_bytes, int* shape, int* xcd, double* ms);

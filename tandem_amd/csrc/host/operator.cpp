@@ -565,17 +565,17 @@ std::vector<double> Operator::autotune_shapes(int ncols, int pb) {
         return std::vector<double>(kSplitOrders * kSplitShapes, -1.0);
     const int saved_variant = variant_, saved_shape = split_shape_[p], saved_xcd = split_xcd_[p];
     const bool saved_auto = split_auto_[p];
-    // the last configuration: the automatic choice, which takes the small applies' shape
+    // the last configuration: the default shape with the small launches, where the rule takes any
     const int last = kSplitOrders * kSplitShapes;
-    const bool small = split_is_small(pb, ncols);
+    bool small = false;
     try {
         variant_ = Variant_Auto;
         time_configs(ncols, pb, last + 1, [&](int c) {
             split_auto_[p] = c == last;
-            if (c == last) return small;
-            split_shape_[p] = c / kSplitOrders;
-            split_xcd_[p] = c % kSplitOrders;
-            return true;
+            split_shape_[p] = c == last ? saved_shape : c / kSplitOrders;
+            split_xcd_[p] = c == last ? saved_xcd : c % kSplitOrders;
+            if (c == last) small = split_small_bits(pb, ncols) != 0;
+            return c < last || small;
         }, ms);
     } catch (...) {
         variant_ = saved_variant;
@@ -591,6 +591,10 @@ std::vector<double> Operator::autotune_shapes(int ncols, int pb) {
     split_shape_[p] = best / kSplitOrders;
     split_xcd_[p] = best % kSplitOrders;
     split_auto_[p] = small && ms[std::size_t(last)] < ms[std::size_t(best)];
+    if (split_auto_[p]) {
+        split_shape_[p] = saved_shape;
+        split_xcd_[p] = saved_xcd;
+    }
     ms.resize(std::size_t(last));
     return ms;
 }
@@ -635,16 +639,11 @@ void Operator::set_split_shape(int pb, int shape, int xcd) {
     split_auto_[pb == 8 ? 0 : 1] = false;
 }
 
-// Launch shape and workgroup order the two-kernel apply of ncols columns runs with.
-void Operator::split_choice(int pb, int ncols, int& shape, int& order) const {
-    const int p = pb == 8 ? 0 : 1;
-    const bool small = split_auto_[p] && split_is_small(pb, ncols);
-    shape = small ? kSplitSmall : split_shape_[p];
-    order = small ? 0 : split_xcd_[p];
-}
-
-bool Operator::split_is_small(int pb, int ncols) const {
-    return int64_t((E_ + 15) / 16) * ncols <= split_small_groups(pb);
+// Which kernels of a two-kernel apply of ncols columns take their small launch.
+int Operator::split_small_bits(int pb, int ncols) const {
+    if (!split_auto_[pb == 8 ? 0 : 1]) return 0;
+    const int64_t facets = pb == 8 ? (s64_ ? s64_->nfacets : 0) : (s32_ ? s32_->nfacets : 0);
+    return split_small(pb, int(Nq_), (facets + 7) / 8 * ncols, int64_t((E_ + 15) / 16) * ncols);
 }
 
 bool Operator::uses_mfma() const {
@@ -1680,6 +1679,7 @@ template <class T> SplitArgs<T> Operator::split_args(DeviceMfma<T> const& m, Dev
     b.num_fgroups = (d.nfacets + 7) / 8;
     b.num_two = d.ntwo;
     b.xcd_remap = 0;
+    b.small = 0;
     b.dot = nullptr;
     return b;
 }
@@ -1715,9 +1715,10 @@ template <class T> void Operator::dispatch(T const* x, T* y, int ncols, int64_t 
         reserve_split(ds, ncols);
         const int64_t ldL = int64_t(E_) * (D_ + 1) * int64_t(block_size());
         SplitArgs<T> sa = split_args(dm, ds);
-        int shape = 0;
-        split_choice(int(sizeof(T)), ncols, shape, sa.xcd_remap);
-        TDG_HIP(launch_elasticity_split<T>(D_, N_, shape, sa, x, y, ds.L.ptr, ncols, ncols > 1 ? ld : 0, ldL,
+        const int p = sizeof(T) == 8 ? 0 : 1;
+        sa.xcd_remap = split_xcd_[p];
+        sa.small = split_small_bits(int(sizeof(T)), ncols);
+        TDG_HIP(launch_elasticity_split<T>(D_, N_, split_shape_[p], sa, x, y, ds.L.ptr, ncols, ncols > 1 ? ld : 0, ldL,
                                            stream_));
     } else if (uses_mfma()) {
         if constexpr (std::is_same<T, double>::value) launch_mfma(*m64_, x, y, ncols, ld);
@@ -1735,8 +1736,10 @@ int64_t Operator::dot_partials_capacity() const {
     if (!(kind_ == Kind_Elasticity && mfma_supported(D_, N_))) return 0;
     const int64_t ng = int64_t((E_ + 15) / 16);
     int64_t m = 0;
-    for (int sh = 0; sh <= kSplitSmall; ++sh)
-        m = std::max({m, split_element_workgroups<double>(sh, ng), split_element_workgroups<float>(sh, ng)});
+    for (int sh = 0; sh < kSplitShapes; ++sh)
+        for (int small : {0, int(kSmallElements)})
+            m = std::max({m, split_element_workgroups<double>(sh, small, ng),
+                          split_element_workgroups<float>(sh, small, ng)});
     return m;
 }
 
@@ -1759,12 +1762,13 @@ template <class T> int64_t Operator::apply_dot_impl(T const* x, T* y, double* pa
         else return *m32_;
     }();
     SplitArgs<T> sa = split_args(dm, ds);
-    int shape = 0;
-    split_choice(int(sizeof(T)), 1, shape, sa.xcd_remap);
+    const int p = sizeof(T) == 8 ? 0 : 1;
+    sa.xcd_remap = split_xcd_[p];
+    sa.small = split_small_bits(int(sizeof(T)), 1);
     sa.dot = partials;
     const int64_t ldL = int64_t(E_) * (D_ + 1) * int64_t(block_size());
-    TDG_HIP(launch_elasticity_split<T>(D_, N_, shape, sa, x, y, ds.L.ptr, 1, 0, ldL, stream_));
-    return split_element_workgroups<T>(shape, int64_t((E_ + 15) / 16));
+    TDG_HIP(launch_elasticity_split<T>(D_, N_, split_shape_[p], sa, x, y, ds.L.ptr, 1, 0, ldL, stream_));
+    return split_element_workgroups<T>(split_shape_[p], sa.small, int64_t((E_ + 15) / 16));
 }
 
 int64_t Operator::apply_dot(double const* x, double* y, double* partials) { return apply_dot_impl(x, y, partials); }
@@ -1808,9 +1812,9 @@ void Operator::apply_noalloc(double const* x, double* y, double* scratch, std::s
         throw std::runtime_error("no kernel compiled for this dimension/degree");
     TDG_HIP(launch_zero_slots<double>(scratch, s64_->idle.ptr, int64_t(s64_->idle.n), int(block_size()), stream_));
     SplitArgs<double> sa = split_args(*m64_, *s64_);
-    int shape = 0;
-    split_choice(8, 1, shape, sa.xcd_remap);
-    TDG_HIP(launch_elasticity_split<double>(D_, N_, shape, sa, x, y, scratch, 1, 0, int64_t(need), stream_));
+    sa.xcd_remap = split_xcd_[0];
+    sa.small = split_small_bits(8, 1);
+    TDG_HIP(launch_elasticity_split<double>(D_, N_, split_shape_[0], sa, x, y, scratch, 1, 0, int64_t(need), stream_));
 }
 void Operator::apply(float const* x, float* y) { dispatch(x, y, 1, 0); }
 void Operator::apply_batched(double const* X, double* Y, int ncols, int64_t ld) { dispatch(X, Y, ncols, ld); }

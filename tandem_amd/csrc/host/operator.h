@@ -347,8 +347,7 @@ private:
     int split_xcd_[2] = {2, 1};
     // whether small applies take the shape made for them instead (until a shape is chosen explicitly)
     bool split_auto_[2] = {true, true};
-    void split_choice(int pb, int ncols, int& shape, int& order) const;
-    bool split_is_small(int pb, int ncols) const;
+    int split_small_bits(int pb, int ncols) const;
     double time_configs(int ncols, int pb, int count, std::function<bool(int)> const& select, std::vector<double>& ms);
 };
 

@@ -19,7 +19,7 @@ TDG_SPLIT_DECL(2, 6)
 template <class T>
 hipError_t launch_elasticity_split(int dim, int degree, int shape, SplitArgs<T> const& a, T const* x, T* y, T* L,
                                    int ncols, int64_t ld, int64_t ldL, hipStream_t s) {
-    if (shape < 0 || shape > kSplitSmall) return hipErrorInvalidValue;
+    if (shape < 0 || shape >= kSplitShapes) return hipErrorInvalidValue;
     if (dim == 3) {
         switch (degree) {
         case 2: return launch_split_d3p2<T>(shape, a, x, y, L, ncols, ld, ldL, s);
@@ -37,11 +37,11 @@ hipError_t launch_elasticity_split(int dim, int degree, int shape, SplitArgs<T> 
     return hipErrorInvalidValue;
 }
 
-template <class T> int64_t split_element_workgroups(int shape, int64_t num_groups) {
-    return split::element_workgroups_of<T>(shape, num_groups);
+template <class T> int64_t split_element_workgroups(int shape, int small, int64_t num_groups) {
+    return split::element_workgroups_of<T>(shape, small, num_groups);
 }
-template int64_t split_element_workgroups<double>(int, int64_t);
-template int64_t split_element_workgroups<float>(int, int64_t);
+template int64_t split_element_workgroups<double>(int, int, int64_t);
+template int64_t split_element_workgroups<float>(int, int, int64_t);
 
 namespace {
 template <class T> __global__ void zero_slots_kernel(T* L, int32_t const* slots, int64_t n, int bs) {

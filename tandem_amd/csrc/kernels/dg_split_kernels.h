@@ -819,6 +819,28 @@ inline int64_t resident_workgroups(void const* k, int threads, int64_t nvb) {
     return cap >= 8 ? std::min(nvb, cap) : nvb;
 }
 
+// Small launches: G groups of 16 elements (8 facets) per workgroup, each shared by as many waves as it
+// has blocks of points (tiles).  A mesh of a few hundred groups otherwise occupies a few CUs with waves
+// that each run one long chain of matrix-core steps.  The results do not depend on G.
+template <int D, int N, class T, int G>
+hipError_t run_small_facets(SplitArgs<T> const& a, T const* x, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
+                            hipStream_t s) {
+    using L = MfmaLayout<D, N>;
+    const int64_t ft = ((a.num_fgroups + G - 1) / G + 7) / 8 * 8 * int64_t(ncols);
+    hipLaunchKernelGGL((elasticity_facet_kernel<D, N, T, G * L::FT, 2, true, false, L::FT>), dim3(unsigned(ft)),
+                       dim3(64 * G * L::FT), 0, s, a, x, Lbuf, ld, ldL, ncols, unsigned(ft));
+    return hipGetLastError();
+}
+template <int D, int N, class T, int G>
+hipError_t run_small_elements(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
+                              hipStream_t s) {
+    using L = MfmaLayout<D, N>;
+    const int64_t et = ((a.num_groups + G - 1) / G + 7) / 8 * 8 * int64_t(ncols);
+    hipLaunchKernelGGL((elasticity_element_kernel<D, N, T, G * L::QB, 2, false, true, false, L::QB>),
+                       dim3(unsigned(et)), dim3(64 * G * L::QB), 0, s, a, x, Lbuf, y, ld, ldL, ncols, unsigned(et));
+    return hipGetLastError();
+}
+
 template <int D, int N, class T, class S>
 hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
                      hipStream_t s) {
@@ -826,62 +848,46 @@ hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols
     const int64_t ft = (fb + 7) / 8 * 8 * int64_t(ncols);
     const int64_t et = element_workgroups<S>(a.num_groups) * int64_t(ncols);
     if (ft > int64_t(0x7fffffff) || et > int64_t(0x7fffffff)) return hipErrorInvalidValue;
-    if (a.xcd_remap == 2) {
-        auto fk = elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, true>;
-        auto ek = elasticity_element_kernel<D, N, T, S::ew, S::eocc, S::deep, S::vtail, true>;
-        if (ft > 0) {
+    const bool persist = a.xcd_remap == 2;
+    hipError_t e = hipSuccess;
+    if (ft > 0) {
+        if (a.small & kSmallFacets) {
+            e = a.num_fgroups * ncols <= kSmallOneGroup
+                    ? run_small_facets<D, N, T, 1>(a, x, Lbuf, ncols, ld, ldL, s)
+                    : run_small_facets<D, N, T, 2>(a, x, Lbuf, ncols, ld, ldL, s);
+        } else if (persist) {
+            auto fk = elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, true>;
             const int64_t fg = resident_workgroups(reinterpret_cast<void const*>(fk), 64 * S::fw, ft);
             hipLaunchKernelGGL(fk, dim3(unsigned(fg)), dim3(64 * S::fw), 0, s, a, x, Lbuf, ld, ldL, ncols,
                                unsigned(ft));
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
+            e = hipGetLastError();
+        } else {
+            hipLaunchKernelGGL((elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, false>),
+                               dim3(unsigned(ft)), dim3(64 * S::fw), 0, s, a, x, Lbuf, ld, ldL, ncols, unsigned(ft));
+            e = hipGetLastError();
         }
+        if (e != hipSuccess) return e;
+    }
+    if (a.small & kSmallElements)
+        return a.num_groups * ncols <= kSmallOneGroup
+                   ? run_small_elements<D, N, T, 1>(a, x, y, Lbuf, ncols, ld, ldL, s)
+                   : run_small_elements<D, N, T, 2>(a, x, y, Lbuf, ncols, ld, ldL, s);
+    if (persist) {
+        auto ek = elasticity_element_kernel<D, N, T, S::ew, S::eocc, S::deep, S::vtail, true>;
         const int64_t eg = resident_workgroups(reinterpret_cast<void const*>(ek), 64 * S::ew, et);
         hipLaunchKernelGGL(ek, dim3(unsigned(eg)), dim3(64 * S::ew), 0, s, a, x, Lbuf, y, ld, ldL, ncols,
                            unsigned(et));
         return hipGetLastError();
-    }
-    if (ft > 0) {
-        hipLaunchKernelGGL((elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, false>), dim3(unsigned(ft)),
-                           dim3(64 * S::fw), 0, s, a, x, Lbuf, ld, ldL, ncols, unsigned(ft));
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL((elasticity_element_kernel<D, N, T, S::ew, S::eocc, S::deep, S::vtail, false>),
                        dim3(unsigned(et)), dim3(64 * S::ew), 0, s, a, x, Lbuf, y, ld, ldL, ncols, unsigned(et));
     return hipGetLastError();
 }
 
-// Small meshes: G groups of 16 elements (8 facets) per workgroup, each shared by as many waves as it has
-// blocks of points (tiles).  A mesh of a few hundred groups otherwise occupies a few CUs with waves that
-// each run one long chain of matrix-core steps.  The results do not depend on G.
-template <int D, int N, class T, int G>
-hipError_t run_small(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
-                     hipStream_t s) {
-    using L = MfmaLayout<D, N>;
-    const int64_t ft = ((a.num_fgroups + G - 1) / G + 7) / 8 * 8 * int64_t(ncols);
-    const int64_t et = ((a.num_groups + G - 1) / G + 7) / 8 * 8 * int64_t(ncols);
-    if (ft > int64_t(0x7fffffff) || et > int64_t(0x7fffffff)) return hipErrorInvalidValue;
-    if (ft > 0) {
-        hipLaunchKernelGGL((elasticity_facet_kernel<D, N, T, G * L::FT, 2, true, false, L::FT>), dim3(unsigned(ft)),
-                           dim3(64 * G * L::FT), 0, s, a, x, Lbuf, ld, ldL, ncols, unsigned(ft));
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL((elasticity_element_kernel<D, N, T, G * L::QB, 2, false, true, false, L::QB>),
-                       dim3(unsigned(et)), dim3(64 * G * L::QB), 0, s, a, x, Lbuf, y, ld, ldL, ncols, unsigned(et));
-    return hipGetLastError();
-}
-inline int64_t small_workgroups(int64_t num_groups) { return (num_groups + 7) / 8 * 8; } // one column: G = 1
-
 // The shape table (index < kSplitShapes): FP64 kernels hold up to two waves per SIMD, FP32 more.
 template <int D, int N, class T>
 hipError_t run_split(int shape, SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
                      hipStream_t s) {
-    if (shape == kSplitSmall)
-        // two groups a workgroup share the tables once every CU has work
-        return a.num_groups * ncols <= kSmallOneGroup ? run_small<D, N, T, 1>(a, x, y, Lbuf, ncols, ld, ldL, s)
-                                                      : run_small<D, N, T, 2>(a, x, y, Lbuf, ncols, ld, ldL, s);
     if constexpr (sizeof(T) == 8) {
         switch (shape) {
         case 0: return run_shape<D, N, T, Shape<4, 2, 8, 2, false, true>>(a, x, y, Lbuf, ncols, ld, ldL, s);
@@ -900,9 +906,9 @@ hipError_t run_split(int shape, SplitArgs<T> const& a, T const* x, T* y, T* Lbuf
     return hipErrorInvalidValue;
 }
 
-template <class T> int64_t element_workgroups_of(int shape, int64_t num_groups) {
-    if (shape == kSplitSmall)
-        return num_groups <= kSmallOneGroup ? small_workgroups(num_groups) : small_workgroups((num_groups + 1) / 2);
+template <class T> int64_t element_workgroups_of(int shape, int small, int64_t num_groups) {
+    if (small & kSmallElements) // (two groups a workgroup above kSmallOneGroup)
+        return ((num_groups <= kSmallOneGroup ? num_groups : (num_groups + 1) / 2) + 7) / 8 * 8;
     if constexpr (sizeof(T) == 8) {
         switch (shape) {
         case 0: return element_workgroups<Shape<4, 2, 8, 2, false, true>>(num_groups);

@@ -98,23 +98,33 @@ template <class T> struct SplitArgs {
     int64_t num_elements, num_groups, num_facets, num_fgroups, num_two;
     int xcd_remap; // workgroup order: 0 linear; 1 one contiguous range of groups per XCD (one column);
                    // 2 as 1, persistent (the resident workgroups loop over the blocks)
+    int small;     // kSmallFacets | kSmallElements: those kernels' waves share each group
     double* dot;   // one column, optional: per element workgroup the partial sum of x . y
 };
 
 // Number of launch shapes of the two-kernel apply (waves per workgroup, occupancy targets, element
 // prefetch depth, lift tail on the vector ALU or the matrix cores), per precision.
 constexpr int kSplitShapes = 4;
-// Launch shape of small applies: the waves of a workgroup share each group of elements (facets), one
-// group a workgroup up to kSmallOneGroup groups x columns, then two.  Taken up to split_small_groups
-// groups of 16 elements x columns.  us per apply, other shapes -> this one, at 24 / 192 / 375 / 648 groups:
-//   3D P4 FP64  70 -> 24, 75 -> 54, 84 -> 73, 94 -> 116     FP32  35 -> 18, 37 -> 36, 45 -> 53, 50 -> 80
-//   3D P3 FP64  35 -> 16, 38 -> 29, 45 -> 38, 53 -> 54      FP32  19 -> 13, 20 -> 18, 25 -> 26, 31 -> 34
-//   3D P2 FP64  18 -> 12, 19 -> 15,  -      , 26 -> 27      FP32  11 -> 10, 12 -> 12,  -      , 15 -> 19
-// (2D P6 and P4 alike; 16 columns of 24 groups: P4 FP64 86 -> 75, FP32 47 -> 53).  Above, the other shapes
-// win: two waves a SIMD share one table and nothing is summed across waves.
-constexpr int kSplitSmall = kSplitShapes;
-constexpr int64_t kSmallOneGroup = 256;
-constexpr int64_t split_small_groups(int precision_bytes) { return precision_bytes == 8 ? 384 : 192; }
+// Small launches of the two kernels: the waves of a workgroup share each group (one block of points or
+// one facet tile each) and sum in LDS, one group a workgroup up to kSmallOneGroup groups x columns, then
+// two.  us per apply, launch shapes -> elements small -> both small, by groups of 16 elements (facet
+// groups of 8: about 4.3 times as many in 3D, 3 in 2D):
+//   3D P4 FP64  24: 70, 29, 24   81: 72, 30, 28   192: 75, 36, 44   375: 83, 48, 74   1029: 113, 110, 172
+//         FP32  24: 35, 23, 18   81: 35, 23, 21   192: 37, 25, 31   375: 44, 35, 54   1029: 75, 68, 116
+//   3D P3 FP64  24: 35, 21, 17   192: 38, 24, 26   648: 53, 42, 54   1029: 65, 63, 79
+//   2D P6 FP64  72: 28, 15, 13   288: 28, 18, 19   512: 33, 24, 27   1152: 43, 47, 53
+//         FP32  72: 15, 12, 11   288: 16, 13, 14   512: 18, 16, 17   1152: 29, 29, 31
+//   16 columns  3D P4 24: FP64 86, 51, 74  FP32 46, 35, 54
+// Above the limits the launch shapes win: two waves a SIMD share one table and nothing is summed across
+// waves.  With one block of points (3D P2, 2D P2 and P3) the small element kernel only spreads the waves
+// over more CUs: 3D P2 FP64 24: 18 -> 14, 648: 27.0 -> 26.3, but FP32 648: 15 -> 17.
+enum { kSmallFacets = 1, kSmallElements = 2 };
+constexpr int64_t kSmallOneGroup = 256, kSmallFacetGroups = 384, kSmallElementGroups = 1024;
+// facet_groups and element_groups: times columns; Nq: volume points.
+constexpr int split_small(int precision_bytes, int Nq, int64_t facet_groups, int64_t element_groups) {
+    return (facet_groups <= kSmallFacetGroups ? kSmallFacets : 0) |
+           (element_groups <= kSmallElementGroups && (Nq > 16 || precision_bytes == 8) ? kSmallElements : 0);
+}
 // Workgroup orders (SplitArgs::xcd_remap) searched with each shape.
 constexpr int kSplitOrders = 3;
 
@@ -126,7 +136,7 @@ template <class T>
 hipError_t launch_elasticity_split(int dim, int degree, int shape, SplitArgs<T> const& a, T const* x, T* y, T* L,
                                    int ncols, int64_t ld, int64_t ldL, hipStream_t stream);
 // Workgroups of the element kernel of launch shape `shape` for one column (a multiple of 8).
-template <class T> int64_t split_element_workgroups(int shape, int64_t num_groups);
+template <class T> int64_t split_element_workgroups(int shape, int small, int64_t num_groups);
 
 // Zeroes the facet slots listed in `slots` (slot s = entries [s bs, (s + 1) bs) of L).
 template <class T> hipError_t launch_zero_slots(T* L, int32_t const* slots, int64_t nslots, int bs, hipStream_t s);

@@ -91,17 +91,18 @@ def test_small_apply_and_explicit_shapes(cuda, D, n, N):
             assert rel_l2(y.double().cpu().numpy(), ref) <= bar, config
 
 
-@pytest.mark.parametrize("D,n,N,cols", [(3, (4, 4, 4), 4, 17), (2, (16, 16), 6, 25), (3, (8, 7, 7), 2, 1)])
+@pytest.mark.parametrize("D,n,N,cols", [(3, (4, 4, 4), 4, 43), (2, (16, 16), 6, 33), (3, (8, 7, 7), 2, 7)])
 def test_small_apply_limits(cuda, D, n, N, cols):
-    """Groups x columns on both sides of the rule (384 FP64, 192 FP32 groups of 16 elements) and of the
-    one-group-a-workgroup limit, batched and singly; a short CG runs the fused dot on the small shape."""
+    """Groups x columns on both sides of the rules (384 facet groups, 1024 element groups) and of the
+    one-group-a-workgroup limit (256), batched and singly; a short CG runs the fused dot on the small
+    launches."""
     import torch
 
     c = Mixed(D, n, N, seed=5)
     X = np.random.default_rng(6).uniform(-1.0, 1.0, (cols, c.n))
     ref = np.stack([c.oracle.apply(x, nthreads=4) for x in X])
     for dt, bar in ((torch.float64, 1e-12), (torch.float32, 1e-5)):
-        for k in sorted({1, min(cols, 7), min(cols, 11), cols - 1 or 1, cols}):
+        for k in sorted({1, 2, 3, 4, 7, min(cols, 11), cols - 1, cols}):
             Xd = torch.from_numpy(X[:k]).to(cuda).to(dt)
             Y = torch.full_like(Xd, float("nan"))
             c.op.apply_batched(Xd, Y)
