@@ -271,15 +271,29 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
 #pragma unroll
                 for (int r = 0; r < Q; ++r) C[r] = acc{0, 0, 0, 0};
                 const int ab = (tc * nq + min(4 * t + tq, nq - 1)) * NbfP;
+                {
+                    // operands one K-step ahead
+                    T av = sT[ab + min(g, Nbf - 1)], b[Q];
 #pragma unroll
-                for (int s = 0; s < KF; ++s) {
-                    const int k = 4 * s + g, kc = min(k, Nbf - 1);
-                    const bool kin = 4 * s + 3 < Nbf || k < Nbf;
-                    const T av = sT[ab + kc];
+                    for (int r = 0; r < Q; ++r) b[r] = U[min(g, Nbf - 1) + r * Nbf];
 #pragma unroll
-                    for (int r = 0; r < Q; ++r) {
-                        const T b = U[kc + r * Nbf];
-                        C[r] = Mma<T>::mma(av, kin ? b : T(0), C[r]);
+                    for (int s = 0; s < KF; ++s) {
+                        const int k = 4 * s + g;
+                        const bool kin = 4 * s + 3 < Nbf || k < Nbf;
+                        T avn = av, bn[Q];
+#pragma unroll
+                        for (int r = 0; r < Q; ++r) bn[r] = b[r];
+                        if (s + 1 < KF) {
+                            const int kn = min(k + 4, Nbf - 1);
+                            avn = sT[ab + kn];
+#pragma unroll
+                            for (int r = 0; r < Q; ++r) bn[r] = U[kn + r * Nbf];
+                        }
+#pragma unroll
+                        for (int r = 0; r < Q; ++r) C[r] = Mma<T>::mma(av, kin ? b[r] : T(0), C[r]);
+                        av = avn;
+#pragma unroll
+                        for (int r = 0; r < Q; ++r) b[r] = bn[r];
                     }
                 }
                 __builtin_amdgcn_s_setprio(0);

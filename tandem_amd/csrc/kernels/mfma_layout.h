@@ -117,13 +117,16 @@ constexpr int kSplitShapes = 4;
 //   16 columns  3D P4 24: FP64 86, 51, 74  FP32 46, 35, 54
 // Above the limits the launch shapes win: two waves a SIMD share one table and nothing is summed across
 // waves.  With one block of points (3D P2, 2D P2 and P3) the small element kernel only spreads the waves
-// over more CUs: 3D P2 FP64 24: 18 -> 14, 648: 27.0 -> 26.3, but FP32 648: 15 -> 17.
+// over more CUs: 3D P2 FP64 24: 18 -> 14, 648: 27.0 -> 26.3, 912: 28.2 -> 28.4, FP32 648: 15 -> 17.
 enum { kSmallFacets = 1, kSmallElements = 2 };
 constexpr int64_t kSmallOneGroup = 256, kSmallFacetGroups = 384, kSmallElementGroups = 1024;
+constexpr int64_t kSmallElementGroups1 = 512; // one block of points, FP64
 // facet_groups and element_groups: times columns; Nq: volume points.
 constexpr int split_small(int precision_bytes, int Nq, int64_t facet_groups, int64_t element_groups) {
     return (facet_groups <= kSmallFacetGroups ? kSmallFacets : 0) |
-           (element_groups <= kSmallElementGroups && (Nq > 16 || precision_bytes == 8) ? kSmallElements : 0);
+           (element_groups <= (Nq > 16 ? kSmallElementGroups : precision_bytes == 8 ? kSmallElementGroups1 : 0)
+                ? kSmallElements
+                : 0);
 }
 // Workgroup orders (SplitArgs::xcd_remap) searched with each shape.
 constexpr int kSplitOrders = 3;
