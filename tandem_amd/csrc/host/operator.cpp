@@ -1714,12 +1714,12 @@ template <class T> void Operator::dispatch(T const* x, T* y, int ncols, int64_t 
         }();
         reserve_split(ds, ncols);
         const int64_t ldL = int64_t(E_) * (D_ + 1) * int64_t(block_size());
-        SplitArgs<T> sa = split_args(dm, ds);
         const int p = sizeof(T) == 8 ? 0 : 1;
+        SplitArgs<T> sa = split_args(dm, ds);
         sa.xcd_remap = split_xcd_[p];
         sa.small = split_small_bits(int(sizeof(T)), ncols);
-        TDG_HIP(launch_elasticity_split<T>(D_, N_, split_shape_[p], sa, x, y, ds.L.ptr, ncols, ncols > 1 ? ld : 0, ldL,
-                                           stream_));
+        TDG_HIP(launch_elasticity_split<T>(D_, N_, split_shape_[p], sa, x, y, ds.L.ptr, ncols, ncols > 1 ? ld : 0,
+                                           ldL, stream_));
     } else if (uses_mfma()) {
         if constexpr (std::is_same<T, double>::value) launch_mfma(*m64_, x, y, ncols, ld);
         else launch_mfma(*m32_, x, y, ncols, ld);

@@ -7,7 +7,7 @@
 // and the two sides of a point trade their traces across a DPP row mirror.  Two-sided facets come
 // first in the facet order, one-sided (Dirichlet or fault boundary) after them; the side-1 columns
 // of a one-sided facet carry nothing.  Everything is computed in the face-0 frame of each side:
-// the element vector of each column is staged in LDS relabelled to face 0
+// the element vector of each column is read relabelled to face 0
 // (U'(k') = x(perm_f(k'))), so one table T0 of face-0 values and reference gradients is the A
 // operand of every trace and every lift whatever the local face numbers of the 16 facets, and the
 // lifted rows are relabelled back (row k' -> element row perm_f(k')) when they are written:
@@ -26,8 +26,15 @@
 // The basis functions of the nodes off a face vanish on it: values and tangential derivatives are
 // contracted over the face's own nodes (15 of 35 at P4), only the normal derivative over all, in the
 // traces and in the lifts.  A P4 wave issues 165 MFMAs instead of 255; the apply went from 489 to
-// 450 us (FP64, 82,944 P4 tetrahedra) and 163 to 154 us (FP32, 48,000).  The kernel is then bound by
-// neither roof (FP64 matrix cores ~35% busy, ~3 TB/s) but by waits at two waves per SIMD.
+// 450 us (FP64, 82,944 P4 tetrahedra) and 163 to 154 us (FP32, 48,000).
+//
+// The element vectors and the slots of the 16 columns lie apart in memory, so they move in 16-byte
+// pieces, consecutive lanes along a vector: a lane per column and entry touched 16 cache lines with
+// every instruction (a quarter of a 64-byte request each), which bound the FP32 kernel (2D P6, 64
+// columns of 18,432 triangles: 620 us in every launch shape, 370 us in pieces; 3D P4 apply 154 -> 133
+// us FP32, 448 -> 433 us FP64).  The vectors are staged as they are; the relabelling is in the offsets
+// of the B operands.  FP64 P4 is then bound by neither roof (matrix cores ~35% busy, ~3 TB/s) but by
+// waits at two waves per SIMD.
 //
 // Element kernel.  One wave owns 16 consecutive elements; the volume term is the element-centric
 // kernel's (reference gradients on the matrix cores, the stress per point in registers, the
@@ -98,6 +105,26 @@ __device__ __forceinline__ void block_of(unsigned w, unsigned nvb, int ncols, in
     lb = ncols > 1 ? (r / unsigned(ncols)) * 8u + xcd : (xcd_remap ? xcd * (nvb / 8u) + r : w);
 }
 
+// Runs f(virtual block, column, block) over the blocks of this workgroup.  MC (several columns): one
+// block for a.cpw consecutive columns, one after another, so that the tables are loaded once and the
+// block's records come from the CU's own cache after the first column.
+template <bool PERSIST, bool MC, class A, class F>
+__device__ __forceinline__ void for_blocks(A const& a, int ncols, unsigned nvb, F&& f) {
+    unsigned col, lb;
+    if constexpr (MC) {
+        block_of(blockIdx.x, nvb, (ncols + a.cpw - 1) / a.cpw, a.xcd_remap, col, lb);
+        const unsigned c0 = col * unsigned(a.cpw), c1 = min(c0 + unsigned(a.cpw), unsigned(ncols));
+#pragma unroll 1
+        for (unsigned c = c0; c < c1; ++c) f(blockIdx.x, c, lb);
+    } else {
+        for (unsigned vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
+            block_of(vb, nvb, ncols, a.xcd_remap, col, lb);
+            f(vb, col, lb);
+            if (!PERSIST) break;
+        }
+    }
+}
+
 // =====================================================================================  facets
 // Column c of a facet wave holds side 0 of facet c (c < 8) or side 1 of facet 15 - c, so that the
 // two sides of a facet sit in lanes j and 15 - j of the same 16-lane row and trade their traces
@@ -116,7 +143,7 @@ __device__ __forceinline__ double mirror16(double v) {
 
 // SPL > 1 (small meshes): SPL consecutive waves share 8 facets, each taking every SPL-th tile, and sum
 // their lifted rows in LDS.
-template <int D, int N, class T, int W, int OCC, bool VTAIL_ON, bool PERSIST, int SPL = 1>
+template <int D, int N, class T, int W, int OCC, bool VTAIL_ON, bool PERSIST, int SPL = 1, bool MC = false>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(OCC)))
 void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __restrict__ Ls, int64_t ld,
                              int64_t ldL, int ncols, unsigned nvb) {
@@ -138,7 +165,10 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
     constexpr bool VTAIL = VTAIL_ON && D == 3 && MT > 1 && TAIL <= 4;
     constexpr int MM = VTAIL ? MT - 1 : MT;
     constexpr int NT = VTAIL ? TAIL : 1;
-    constexpr int NI = (BS + 3) / 4; // staging steps of 4 entries per column
+    // element vectors and slots move in pieces of 16 bytes: NCK a column, piece i of the wave = 64 o + lane;
+    // a column's last piece ends with its vector (it overlaps the one before it)
+    constexpr int VW = 16 / int(sizeof(T)), NCK = (BS + VW - 1) / VW, NPC = (16 * NCK + 63) / 64;
+    using vec = T __attribute__((ext_vector_type(VW), aligned(sizeof(T))));
 
     __shared__ T sT[NF * nq * NbfP];
     __shared__ int sP[2 * NF * Nbf];
@@ -162,13 +192,11 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
     }
     __syncthreads();
 
-    auto block = [&](unsigned vb) {
-        const int tid = int(threadIdx.x), wv = tid >> 6, lane = lane_of<PERSIST>(tid), j = lane & 15, g = lane >> 4;
+    auto block = [&](unsigned col, unsigned lb) {
+        const int tid = int(threadIdx.x), wv = tid >> 6, lane = lane_of<PERSIST || MC>(tid), j = lane & 15, g = lane >> 4;
         // this lane's column: facet fl, side sd
         const int fl = column_facet(j), sd = j < 8 ? 0 : 1;
         T* const X = sX[wv];
-        unsigned col, lb;
-        block_of(vb, nvb, ncols, a.xcd_remap, col, lb);
         const int part = SPL > 1 ? wv % SPL : 0;
         const int64_t grp = int64_t(lb) * (W / SPL) + wv / SPL;
         const bool live = grp < a.num_fgroups; // uniform per wave
@@ -199,21 +227,21 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
         T rc[DD + 2];
         load_rec(part, rc);
 
-        // element vector of this column in LDS, relabelled to face 0: U'(k', r) = x(perm_f(k'), r);
-        // lane (j, g) moves entries 4 i + g
+        // the 16 element vectors in LDS (zero for columns without a side)
         {
-            T v[NI];
-            T const* xe = x + int64_t(el) * BS + g;
+            vec v[NPC];
 #pragma unroll
-            for (int i = 0; i < NI; ++i) v[i] = (4 * i + 3 < BS || 4 * i + g < BS) ? xe[4 * i] : T(0);
-            int const* const ip = sP + NF * Nbf + lf * Nbf;
+            for (int o = 0; o < NPC; ++o) {
+                const int i = min(64 * o + lane, 16 * NCK - 1), c = i / NCK, at = min((i - c * NCK) * VW, BS - VW);
+                const int ec = __shfl(ok ? el : -1, c, 64);
+                v[o] = *reinterpret_cast<vec const*>(x + int64_t(max(ec, 0)) * BS + at);
+                if (ec < 0) v[o] = vec(T(0));
+            }
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int rem = 4 * i + g;
-                if (4 * i + 3 < BS || rem < BS) {
-                    const int r = rem / Nbf, k = rem - r * Nbf;
-                    X[j * BSP + ip[k] + r * Nbf] = ok ? v[i] : T(0);
-                }
+            for (int o = 0; o < NPC; ++o) {
+                const int i = min(64 * o + lane, 16 * NCK - 1), c = i / NCK, at = min((i - c * NCK) * VW, BS - VW);
+#pragma unroll
+                for (int n = 0; n < VW; ++n) X[c * BSP + at + n] = v[o][n];
             }
         }
         wave_sync(); // staged vectors ready (the region is this wave's)
@@ -232,7 +260,12 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
         if (live) {
             const int tq = mfma_group<T>(j);
             const int tc = min(mfma_reg<T>(j), D);
+            // B operands: U'(k') = x(perm_f(k')); the offsets of the four-channel tiles' K-steps are kept
             T const* const U = X + j * BSP;
+            int const* const pu = sP + lf * Nbf;
+            int uo[KF];
+#pragma unroll
+            for (int s = 0; s < KF; ++s) uo[s] = pu[min(4 * s + g, Nbf - 1)];
             // part of the normal derivative from the nodes off the face, four tiles at a time:
             // register i = point 4 (4 b + i) + g of block b, this lane's point in tile 4 b + i
             acc off[Q];
@@ -260,9 +293,10 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
                         const int k = 4 * s + g, kc = min(k, Nbf - 1);
                         const bool kin = 4 * s + 3 < Nbf || k < Nbf;
                         const T av = sT[ab + kc];
+                        const int un = pu[kc];
 #pragma unroll
                         for (int r = 0; r < Q; ++r) {
-                            const T b = U[kc + r * Nbf];
+                            const T b = U[un + r * Nbf];
                             off[r] = Mma<T>::mma(av, kin ? b : T(0), off[r]);
                         }
                     }
@@ -275,7 +309,7 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
                     // operands one K-step ahead
                     T av = sT[ab + min(g, Nbf - 1)], b[Q];
 #pragma unroll
-                    for (int r = 0; r < Q; ++r) b[r] = U[min(g, Nbf - 1) + r * Nbf];
+                    for (int r = 0; r < Q; ++r) b[r] = U[uo[0] + r * Nbf];
 #pragma unroll
                     for (int s = 0; s < KF; ++s) {
                         const int k = 4 * s + g;
@@ -284,10 +318,9 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
 #pragma unroll
                         for (int r = 0; r < Q; ++r) bn[r] = b[r];
                         if (s + 1 < KF) {
-                            const int kn = min(k + 4, Nbf - 1);
-                            avn = sT[ab + kn];
+                            avn = sT[ab + min(k + 4, Nbf - 1)];
 #pragma unroll
-                            for (int r = 0; r < Q; ++r) bn[r] = U[kn + r * Nbf];
+                            for (int r = 0; r < Q; ++r) bn[r] = U[uo[s + 1] + r * Nbf];
                         }
 #pragma unroll
                         for (int r = 0; r < Q; ++r) C[r] = Mma<T>::mma(av, kin ? b[r] : T(0), C[r]);
@@ -480,26 +513,32 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
         }
         if constexpr (SPL == 1) wave_sync();
         else __syncthreads();
-        if (ok) {
-            T* const dst = Lc + (int64_t(el) * NF + lf) * BS + g;
+        {
+            const int slot = ok ? el * NF + lf : -1;
+            int ln = lane; // opaque: the pieces' places are computed again, not held across the tile loop
+            __asm__ volatile("" : "+v"(ln));
+            ln &= 63;
 #pragma unroll
-            for (int ii = 0; ii < (NI + SPL - 1) / SPL; ++ii) {
-                const int i = SPL * ii + part;
-                if (4 * i + 3 < BS || 4 * i + g < BS) {
-                    T v = sX[wv - part][j * BSP + 4 * i + g];
+            for (int oo = 0; oo < (NPC + SPL - 1) / SPL; ++oo) {
+                const int i = 64 * (SPL * oo + part) + ln;
+                const int ic = min(i, 16 * NCK - 1), c = ic / NCK, at = min((ic - c * NCK) * VW, BS - VW);
+                const int sc = __shfl(slot, c, 64);
+                if (i < 16 * NCK && sc >= 0) {
+                    vec v;
 #pragma unroll
-                    for (int s = 1; s < SPL; ++s) v += sX[wv - part + s][j * BSP + 4 * i + g];
-                    dst[4 * i] = v;
+                    for (int n = 0; n < VW; ++n) {
+                        T w = sX[wv - part][c * BSP + at + n];
+#pragma unroll
+                        for (int s = 1; s < SPL; ++s) w += sX[wv - part + s][c * BSP + at + n];
+                        v[n] = w;
+                    }
+                    *reinterpret_cast<vec*>(Lc + int64_t(sc) * BS + at) = v;
                 }
             }
         }
         wave_sync(); // every read of the staged region is done before the next block restages it
     };
-    if constexpr (PERSIST) {
-        for (unsigned vb = blockIdx.x; vb < nvb; vb += gridDim.x) block(vb);
-    } else {
-        block(blockIdx.x);
-    }
+    for_blocks<PERSIST, MC>(a, ncols, nvb, [&](unsigned, unsigned col, unsigned lb) { block(col, lb); });
 }
 
 // =====================================================================================  elements
@@ -509,7 +548,7 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
 // the slots are read at the end; the other waves of the SIMD cover the waits.
 // SPL > 1 (small meshes): SPL consecutive waves share 16 elements, each taking every SPL-th block of
 // points, and sum their results from LDS as they store them.
-template <int D, int N, class T, int W, int OCC, bool DEEP, bool VTAIL_ON, bool PERSIST, int SPL = 1>
+template <int D, int N, class T, int W, int OCC, bool DEEP, bool VTAIL_ON, bool PERSIST, int SPL = 1, bool MC = false>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(OCC)))
 void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const* __restrict__ Ls,
                                T* __restrict__ ys, int64_t ld, int64_t ldL, int ncols, unsigned nvb) {
@@ -523,8 +562,14 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
     constexpr bool VTAIL = VTAIL_ON && D == 3 && MT > 1 && TAIL <= 4;
     constexpr int MM = VTAIL ? MT - 1 : MT;
     constexpr int NT = VTAIL ? TAIL : 1;
-    constexpr int NX = (16 * BS + 63) / 64;      // staged entries per lane
-    constexpr int NO = (NX + SPL - 1) / SPL;     // output entries per lane: 64 (SPL o + part) + lane
+    // vectors and slots move in pieces of up to 16 bytes, NCK an element: piece i of the wave = 64 o + lane;
+    // an element's last piece ends with its vector (it may overlap the one before it).  The wave's data are
+    // contiguous, so in FP32 pieces off their alignment buy nothing: 3D P4 (105 entries), 48,000 elements,
+    // 135 us in overlapping 16-byte pieces, 133 us in single entries; FP64, 82,944: 434 us and 440 us.
+    constexpr int VW = sizeof(T) == 8 ? 2 : BS % 4 == 0 ? 4 : BS % 2 == 0 ? 2 : 1;
+    constexpr int NCK = (BS + VW - 1) / VW, NPC = (16 * NCK + 63) / 64;
+    constexpr int NO = (NPC + SPL - 1) / SPL; // output pieces per lane: 64 (SPL o + part) + lane
+    using vec = T __attribute__((ext_vector_type(VW), aligned(sizeof(T))));
     static_assert(W % SPL == 0 && (SPL == 1 || (SPL <= QB && !PERSIST && !DEEP)), "whole groups of waves");
 
     __shared__ T sV[D * Nq * NbfP];
@@ -538,11 +583,9 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
     }
     __syncthreads();
 
-    auto block = [&](unsigned vb) {
-        const int tid = int(threadIdx.x), wv = tid >> 6, lane = lane_of<PERSIST>(tid), j = lane & 15, g = lane >> 4;
+    auto block = [&](unsigned vb, unsigned col, unsigned lb) {
+        const int tid = int(threadIdx.x), wv = tid >> 6, lane = lane_of<PERSIST || MC>(tid), j = lane & 15, g = lane >> 4;
         T* const U = sU[wv];
-        unsigned col, lb;
-        block_of(vb, nvb, ncols, a.xcd_remap, col, lb);
         const int part = SPL > 1 ? wv % SPL : 0;
         const int64_t grp = int64_t(lb) * (W / SPL) + wv / SPL;
         const bool live = grp < a.num_groups; // uniform per wave
@@ -554,7 +597,6 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         const bool valid = j < nel;
         const int64_t gj = live ? grp : 0;
         T const* const xw = x + (live ? e0 : 0) * BS; // this wave's 16 element vectors (contiguous)
-        const int nout = nel * BS;
 
         // point data of point q = 16 b + mfma_row(g, i) (clamped), for registers i0 <= i < i1
         auto load_pd = [&](int b, T (&pd)[4][NCH], int i0 = 0, int i1 = 4) {
@@ -566,17 +608,23 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
                 for (int c = 0; c < NCH; ++c) pd[i][c] = vd[c * 16];
             }
         };
-        // the element's facet slots for output entry i0 + lane (16 consecutive elements: contiguous)
+        // place of piece i: element c, first entry at (pieces past the wave's last repeat that one)
+        auto place = [&](int i, int& c, int& at) {
+            const int ic = min(i, 16 * NCK - 1);
+            c = ic / NCK;
+            at = min((ic - c * NCK) * VW, BS - VW);
+        };
+        // sums of the element's facet slots for the output pieces
         T const* const lsl = Lc + (live ? e0 : 0) * NF * BS;
-        auto load_slots = [&](T (&ls)[NO]) {
+        auto load_slots = [&](vec (&ls)[NO], int ln) {
 #pragma unroll
             for (int o = 0; o < NO; ++o) {
-                const int i = 64 * (SPL * o + part) + lane;
-                const int ic = min(i, max(nout - 1, 0));
-                const int jj = ic / BS, rem = ic - jj * BS;
-                T v = T(0);
+                int c, at;
+                place(64 * (SPL * o + part) + ln, c, at);
+                T const* const p = lsl + min(c, max(nel - 1, 0)) * NF * BS + at;
+                vec v = *reinterpret_cast<vec const*>(p);
 #pragma unroll
-                for (int f = 0; f < NF; ++f) v += lsl[(jj * NF + f) * BS + rem];
+                for (int f = 1; f < NF; ++f) v += *reinterpret_cast<vec const*>(p + f * BS);
                 ls[o] = v;
             }
         };
@@ -585,13 +633,19 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         if constexpr (DEEP) load_pd(0, pd);
         if (live) {
             // every load first (clamped addresses), then the LDS stores: no load waits on another
-            T v[NX];
+            vec v[NPC];
 #pragma unroll
-            for (int o = 0; o < NX; ++o) v[o] = xw[min(64 * o + lane, nout - 1)];
+            for (int o = 0; o < NPC; ++o) {
+                int c, at;
+                place(64 * o + lane, c, at);
+                v[o] = *reinterpret_cast<vec const*>(xw + min(c, nel - 1) * BS + at);
+            }
 #pragma unroll
-            for (int o = 0; o < NX; ++o) {
-                const int i = 64 * o + lane;
-                if (i < 16 * BS) U[(i / BS) * BSP + i % BS] = i < nout ? v[o] : T(0);
+            for (int o = 0; o < NPC; ++o) {
+                int c, at;
+                place(64 * o + lane, c, at);
+#pragma unroll
+                for (int n = 0; n < VW; ++n) U[c * BSP + at + n] = c < nel ? v[o][n] : T(0);
             }
         }
         wave_sync(); // staged vectors ready (the region is this wave's)
@@ -607,7 +661,12 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         for (int kt = 0; kt < NT; ++kt)
 #pragma unroll
             for (int u = 0; u < Q; ++u) Yt[kt][u] = T(0);
-        T ls[NO];
+        vec ls[NO];
+        int ln = lane;
+        if constexpr (VW > 1) { // opaque: the pieces' places are computed again, not held across the volume loop
+            __asm__ volatile("" : "+v"(ln));
+            ln &= 63;
+        }
 
         // late: the point data of registers 2 and 3 are loaded here, once the block's reference
         // gradients are on the matrix cores
@@ -703,7 +762,7 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
                 for (int b = 0; b < QB; ++b) {
                     T pn[4][NCH];
                     if (b + 1 < QB) load_pd(b + 1, pn);
-                    else load_slots(ls);
+                    else load_slots(ls, ln);
                     volume_block(b, pd, false);
                     if (b + 1 < QB) {
 #pragma unroll
@@ -757,31 +816,44 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
                         for (int u = 0; u < Q; ++u) U[j * BSP + 16 * MM + kt + u * Nbf] = Yt[kt][u];
                 }
             }
-            if constexpr (!DEEP) load_slots(ls);
+            if constexpr (!DEEP) load_slots(ls, ln);
         }
         // x again for x . y (one column only: Krylov solvers), all loads issued before the first use
-        T xv[NO];
+        vec xv[NO];
         if (a.dot && live) {
 #pragma unroll
-            for (int o = 0; o < NO; ++o) xv[o] = xw[min(64 * (SPL * o + part) + lane, nout - 1)];
+            for (int o = 0; o < NO; ++o) {
+                int c, at;
+                place(64 * (SPL * o + part) + ln, c, at);
+                xv[o] = *reinterpret_cast<vec const*>(xw + min(c, nel - 1) * BS + at);
+            }
         }
         if constexpr (SPL == 1) wave_sync();
         else __syncthreads();
         double dot = 0.0;
         if (live) {
             // y = volume + the element's facet slots
-            T* dst = y + e0 * BS;
+            T* const dst = y + e0 * BS;
 #pragma unroll
             for (int o = 0; o < NO; ++o) {
-                const int i = 64 * (SPL * o + part) + lane;
-                if (i < nout) {
-                    const int jj = i / BS, rem = i - jj * BS;
-                    T v = sU[wv - part][jj * BSP + rem];
+                const int i = 64 * (SPL * o + part) + ln;
+                int c, at;
+                place(i, c, at);
+                if (i < 16 * NCK && c < nel) {
+                    vec v;
 #pragma unroll
-                    for (int s = 1; s < SPL; ++s) v += sU[wv - part + s][jj * BSP + rem];
-                    v += ls[o];
-                    dst[i] = v;
-                    if (a.dot) dot += double(xv[o]) * double(v);
+                    for (int n = 0; n < VW; ++n) {
+                        T w = sU[wv - part][c * BSP + at + n];
+#pragma unroll
+                        for (int s = 1; s < SPL; ++s) w += sU[wv - part + s][c * BSP + at + n];
+                        v[n] = w + ls[o][n];
+                    }
+                    *reinterpret_cast<vec*>(dst + c * BS + at) = v;
+                    if (a.dot) {
+#pragma unroll
+                        for (int n = 0; n < VW; ++n) // the overlap of the last piece counts once
+                            if (BS % VW == 0 || at + n >= (i - c * NCK) * VW) dot += double(xv[o][n]) * double(v[n]);
+                    }
                 }
             }
         }
@@ -801,11 +873,7 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         }
         wave_sync(); // every read of the staged region is done before the next block restages it
     };
-    if constexpr (PERSIST) {
-        for (unsigned vb = blockIdx.x; vb < nvb; vb += gridDim.x) block(vb);
-    } else {
-        block(blockIdx.x);
-    }
+    for_blocks<PERSIST, MC>(a, ncols, nvb, block);
 }
 
 // Launch shapes of the two kernels, searched by the autotuner: waves per workgroup and the
@@ -855,6 +923,14 @@ hipError_t run_small_elements(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, 
     return hipGetLastError();
 }
 
+// Columns a workgroup takes one after another (its tables loaded once, its records in the CU's cache):
+// at most 8, fewer where the chip would otherwise get too few workgroups to finish evenly.  us per apply of
+// 64 columns with 1 / 4 / 8 / 16 a visit: 2D P6 FP32 18,432 elements 758 / 720 / 721 / 755, 80,000: 3356 / 3174 /
+// 3117 / 3162; 3D P4 FP64 6,000: 2291 / 2136 / 2427 / 2518, 24,576: 9185 / 8496 / 8308 / 8297.
+inline int columns_per_visit(int64_t blocks, int ncols) {
+    return int(std::max<int64_t>(1, std::min<int64_t>({8, ncols, blocks * ncols / 8192})));
+}
+
 template <int D, int N, class T, class S>
 hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
                      hipStream_t s) {
@@ -869,6 +945,13 @@ hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols
             e = a.num_fgroups * ncols <= kSmallOneGroup
                     ? run_small_facets<D, N, T, 1>(a, x, Lbuf, ncols, ld, ldL, s)
                     : run_small_facets<D, N, T, 2>(a, x, Lbuf, ncols, ld, ldL, s);
+        } else if (ncols > 1) {
+            SplitArgs<T> m = a;
+            m.cpw = columns_per_visit(ft / ncols, ncols);
+            const int64_t gf = ft / ncols * ((ncols + m.cpw - 1) / m.cpw);
+            hipLaunchKernelGGL((elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, false, 1, true>),
+                               dim3(unsigned(gf)), dim3(64 * S::fw), 0, s, m, x, Lbuf, ld, ldL, ncols, unsigned(gf));
+            e = hipGetLastError();
         } else if (persist) {
             auto fk = elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, true>;
             const int64_t fg = resident_workgroups(reinterpret_cast<void const*>(fk), 64 * S::fw, ft);
@@ -886,6 +969,14 @@ hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols
         return a.num_groups * ncols <= kSmallOneGroup
                    ? run_small_elements<D, N, T, 1>(a, x, y, Lbuf, ncols, ld, ldL, s)
                    : run_small_elements<D, N, T, 2>(a, x, y, Lbuf, ncols, ld, ldL, s);
+    if (ncols > 1) {
+        SplitArgs<T> m = a;
+        m.cpw = columns_per_visit(et / ncols, ncols);
+        const int64_t ge = et / ncols * ((ncols + m.cpw - 1) / m.cpw);
+        hipLaunchKernelGGL((elasticity_element_kernel<D, N, T, S::ew, S::eocc, S::deep, S::vtail, false, 1, true>),
+                           dim3(unsigned(ge)), dim3(64 * S::ew), 0, s, m, x, Lbuf, y, ld, ldL, ncols, unsigned(ge));
+        return hipGetLastError();
+    }
     if (persist) {
         auto ek = elasticity_element_kernel<D, N, T, S::ew, S::eocc, S::deep, S::vtail, true>;
         const int64_t eg = resident_workgroups(reinterpret_cast<void const*>(ek), 64 * S::ew, et);

@@ -98,6 +98,7 @@ template <class T> struct SplitArgs {
     int64_t num_elements, num_groups, num_facets, num_fgroups, num_two;
     int xcd_remap; // workgroup order: 0 linear; 1 one contiguous range of groups per XCD (one column);
                    // 2 as 1, persistent (the resident workgroups loop over the blocks)
+    int cpw;       // several columns: columns a workgroup takes one after another (set by the launch)
     int small;     // kSmallFacets | kSmallElements: those kernels' waves share each group
     double* dot;   // one column, optional: per element workgroup the partial sum of x . y
 };
