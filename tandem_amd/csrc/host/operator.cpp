@@ -836,10 +836,11 @@ template <class T> void Operator::upload_split(DeviceSplit<T>& ds) {
 }
 
 bool Operator::uses_poisson_mfma(int pb, int ncols) const {
+    if (kind_ != Kind_Poisson || variant_ != Variant_Auto ||
+        int64_t(local_size()) * ncols < poisson_mfma_unknowns(int(D_), pb) || (D_ == 2 && N_ == 1))
+        return false;
     int kq = 0, kf = 0;
-    return kind_ == Kind_Poisson && variant_ == Variant_Auto && kernel_rule_sizes(D_, N_, &kq, &kf) == 0 &&
-           kq == int(Nq_) && kf == int(nq_) && !(D_ == 2 && N_ == 1) &&
-           int64_t(local_size()) * ncols >= poisson_mfma_unknowns(int(D_), pb);
+    return kernel_rule_sizes(D_, N_, &kq, &kf) == 0 && kq == int(Nq_) && kf == int(nq_);
 }
 
 template <class T> DevicePoisson<T>& Operator::device_poisson() {

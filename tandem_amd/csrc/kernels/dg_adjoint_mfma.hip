@@ -20,6 +20,9 @@
 // transposed material basis, the facet relabellings, and per wave the 16 u and psi vectors (later the
 // nodal sensitivities, their projections and the output staging).  The number of waves per
 // workgroup is the largest (up to 8) whose LDS fits one CU.
+//
+// Values on a face, and in FP32 its tangential derivatives, are contracted over the face's own nodes only
+// (15 of 35 at P4): 2450 -> 1848 MFMAs a wave at P4, 24,576 tetrahedra in FP32 177 -> 153 us.
 #include "kernels.h"
 #include "mfma_layout.h"
 #include "mfma_ops.h"
@@ -59,6 +62,10 @@ __global__ __launch_bounds__((64 * GradShape<D, N, T>::waves)) void material_gra
     using acc = typename Mma<T>::acc;
     constexpr int Nbf = L::Nbf, Nq = L::Nq, nq = L::nq, Q = D, BS = Nbf * Q, DD = D * D, NF = D + 1;
     constexpr int KS = L::KS, QB = L::QB, MT = L::MT, FT = L::FT, NCH = L::NCH, NFC = L::NFC;
+    // trace K-steps of the four-channel tiles (the rule of the apply's facet kernel; FP64 has no registers for
+    // the held part: 3D P4 would spill), and of the values, which involve the face's own nodes only
+    constexpr bool SPLITK = sizeof(T) == 4 && (FT - (FT + 3) / 4) * (KS - L::KF) >= 5;
+    constexpr int KF = SPLITK ? L::KF : KS, KV = L::KF;
     constexpr int W = S::waves, NV = (FT + 3) / 4; // neighbour value tiles of 16 facet points
     constexpr int nV = S::nV, nT = S::nT, nE = S::nE;
 
@@ -221,21 +228,19 @@ __global__ __launch_bounds__((64 * GradShape<D, N, T>::waves)) void material_gra
             const int nbface = (info.x >> 4) & 3;
             const bool skel = kind == 1;
             const int64_t nb = skel ? int64_t(info.y) : 0;
-            int po[KS], pn[KS];
+            int po[KF], pn[KV];
 #pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                const int kc = min(4 * s + gq, Nbf - 1);
-                po[s] = sP[f * Nbf + kc];
-                pn[s] = sP[nbface * Nbf + kc];
-            }
+            for (int s = 0; s < KF; ++s) po[s] = sP[f * Nbf + min(4 * s + gq, Nbf - 1)];
+#pragma unroll
+            for (int s = 0; s < KV; ++s) pn[s] = sP[nbface * Nbf + min(4 * s + gq, Nbf - 1)];
             // neighbour value traces of u and psi (B operands gathered into registers)
             acc Vn[2][NV][Q];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 T const* X = (h == 0 ? u : psi) + nb * BS;
-                T Nb[KS][Q];
+                T Nb[KV][Q];
 #pragma unroll
-                for (int s = 0; s < KS; ++s) {
+                for (int s = 0; s < KV; ++s) {
                     const int k = 4 * s + gq;
                     const bool kin = 4 * s + 3 < Nbf || k < Nbf;
 #pragma unroll
@@ -250,7 +255,7 @@ __global__ __launch_bounds__((64 * GradShape<D, N, T>::waves)) void material_gra
                     for (int r = 0; r < Q; ++r) Vn[h][v][r] = acc{0, 0, 0, 0};
                     const int ab = min(16 * v + vq, nq - 1) * Nbf; // value channel
 #pragma unroll
-                    for (int s = 0; s < KS; ++s) {
+                    for (int s = 0; s < KV; ++s) {
                         const T av = sTab[ab + min(4 * s + gq, Nbf - 1)];
 #pragma unroll
                         for (int r = 0; r < Q; ++r) Vn[h][v][r] = Mma<T>::mma(av, Nb[s][r], Vn[h][v][r]);
@@ -262,6 +267,7 @@ __global__ __launch_bounds__((64 * GradShape<D, N, T>::waves)) void material_gra
             for (int m = 0; m < MT; ++m) il[m] = sP[NF * Nbf + f * Nbf + min(16 * m + j, Nbf - 1)];
             T const* const fdf = a.FD + ((gj * NF + f) * nq) * NFC * 16 + j;
             T gd = T(0);
+            acc off[2][Q]; // normal derivative from the nodes off the face, four tiles at a time
 #pragma unroll 1
             for (int t = 0; t < FT; ++t) {
                 const int q = 4 * t + gq, qc = min(q, nq - 1);
@@ -275,9 +281,27 @@ __global__ __launch_bounds__((64 * GradShape<D, N, T>::waves)) void material_gra
                 acc Cu[Q], Cp[Q];
 #pragma unroll
                 for (int r = 0; r < Q; ++r) Cu[r] = Cp[r] = acc{0, 0, 0, 0};
+                if (SPLITK && t % 4 == 0) {
+#pragma unroll
+                    for (int r = 0; r < Q; ++r) off[0][r] = off[1][r] = acc{0, 0, 0, 0};
+                    const int ab = (D * nq + min(4 * (t + mfma_reg<T>(j)) + tq, nq - 1)) * Nbf;
+#pragma unroll
+                    for (int s = KF; s < KS; ++s) {
+                        const int k = 4 * s + gq, kc = min(k, Nbf - 1);
+                        const bool kin = 4 * s + 3 < Nbf || k < Nbf;
+                        const T av = sTab[ab + kc];
+                        const int pk = sP[f * Nbf + kc];
+#pragma unroll
+                        for (int r = 0; r < Q; ++r) {
+                            const T bu = Uj[pk + r * Nbf], bp = Pj[pk + r * Nbf];
+                            off[0][r] = Mma<T>::mma(av, kin ? bu : T(0), off[0][r]);
+                            off[1][r] = Mma<T>::mma(av, kin ? bp : T(0), off[1][r]);
+                        }
+                    }
+                }
                 const int ab = (tc * nq + min(4 * t + tq, nq - 1)) * Nbf;
 #pragma unroll
-                for (int s = 0; s < KS; ++s) {
+                for (int s = 0; s < KF; ++s) {
                     const int k = 4 * s + gq;
                     const bool kin = 4 * s + 3 < Nbf || k < Nbf;
                     const T av = sTab[ab + min(k, Nbf - 1)];
@@ -286,6 +310,15 @@ __global__ __launch_bounds__((64 * GradShape<D, N, T>::waves)) void material_gra
                         const T bu = Uj[po[s] + r * Nbf], bp = Pj[po[s] + r * Nbf];
                         Cu[r] = Mma<T>::mma(av, kin ? bu : T(0), Cu[r]);
                         Cp[r] = Mma<T>::mma(av, kin ? bp : T(0), Cp[r]);
+                    }
+                }
+                if constexpr (SPLITK) {
+#pragma unroll
+                    for (int r = 0; r < Q; ++r) {
+                        Cu[r][D] += off[0][r][0];
+                        Cp[r][D] += off[1][r][0];
+                        off[0][r] = acc{off[0][r][1], off[0][r][2], off[0][r][3], 0};
+                        off[1][r] = acc{off[1][r][1], off[1][r][2], off[1][r][3], 0};
                     }
                 }
                 // this lane: facet point q; register c = value (0) / d/dxi_e (1 + e)
