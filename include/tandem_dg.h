@@ -92,7 +92,8 @@ int tdg_mult_f32(tdg_op* op, float const* x, float* y);
  * reference.  The facet slots of the two-kernel apply live in a fixed 64 MiB device array of the
  * library (each GPU holds it until the process ends): operators whose slots need more
  * (elements x (dim+1) x block size doubles > 2^23, about 20,000 P4 tetrahedra) are rejected with
- * TDG_ERR_ARG.  The operator must be on the device already (tdg_upload, which also sets up the array
+ * TDG_ERR_ARG.  Poisson operators large enough for the matrix-core apply keep its traces there where they
+ * fit and otherwise run the kernel that needs none.  The operator must be on the device already (tdg_upload, which also sets up the array
  * on the current device, or one tdg_mult), else TDG_ERR_STATE; with TDG_VARIANT_ASSEMBLED it must
  * have been assembled (tdg_assemble or one tdg_mult), and the apply then uses no scratch memory.  All calls on one GPU share the
  * array: calls that overlap in time on one GPU race; calls ordered on one stream do not. */
@@ -107,7 +108,8 @@ int tdg_set_stream(tdg_op* op, void* stream);
 /* Kernel choice: TDG_VARIANT_AUTO (default) runs the two-kernel matrix-core (MFMA) apply where one
  * is compiled for the operator (elasticity, 3D P2-P4, 2D P2-P4 and P6): a facet kernel evaluates each
  * facet once (both sides' traces, the flux and both lifts) into per-element-face slots, an element
- * kernel applies the volume term and adds the slots; the thread-per-point kernel otherwise.
+ * kernel applies the volume term and adds the slots; for Poisson (except 2D P1), above a size rule, its
+ * matrix-core apply (own traces, then elements); the thread-per-point kernel otherwise.
  * TDG_VARIANT_POINTS always runs the thread-per-point kernel.  TDG_VARIANT_MFMA_ELEMENT runs the
  * element-centric MFMA kernel (each element evaluates both sides of its faces, as the reference's
  * element loop does), TDG_VARIANT_MFMA_XCD the same kernel with its workgroups renumbered so that

@@ -481,8 +481,8 @@ void Operator::reserve_columns(int ncols) {
         reserve_split(*s64_, ncols);
         reserve_split(*s32_, ncols);
     }
-    if (uses_poisson_mfma(8, ncols)) reserve_poisson(device_poisson<double>(), ncols);
-    if (uses_poisson_mfma(4, ncols)) reserve_poisson(device_poisson<float>(), ncols);
+    if (uses_poisson_mfma(8, ncols)) reserve_poisson(device_poisson<double>(), poisson_columns(8, ncols));
+    if (uses_poisson_mfma(4, ncols)) reserve_poisson(device_poisson<float>(), poisson_columns(4, ncols));
 }
 
 template <class T> void Operator::reserve_split(DeviceSplit<T>& ds, int ncols) {
@@ -843,6 +843,12 @@ bool Operator::uses_poisson_mfma(int pb, int ncols) const {
     return kernel_rule_sizes(D_, N_, &kq, &kf) == 0 && kq == int(Nq_) && kf == int(nq_);
 }
 
+// Columns a matrix-core Poisson apply takes at a time: its traces (about four vectors a column) stay within
+// 1 GiB, or one column's.
+int Operator::poisson_columns(int pb, int ncols) const {
+    return int(std::max<int64_t>(1, std::min<int64_t>(ncols, (int64_t(1) << 30) / int64_t(trace_entries() * pb))));
+}
+
 template <class T> DevicePoisson<T>& Operator::device_poisson() {
     auto& slot = [&]() -> auto& {
         if constexpr (std::is_same<T, double>::value) return p64_;
@@ -924,8 +930,9 @@ template <class T> void Operator::upload_poisson(DevicePoisson<T>& d) {
 
 template <class T> void Operator::launch_poisson_device(T const* x, T* y, T* TR, int ncols, int64_t ld) {
     DevicePoisson<T>& d = device_poisson<T>();
+    const int range = poisson_columns(int(sizeof(T)), ncols);
     if (!TR) {
-        reserve_poisson(d, ncols);
+        reserve_poisson(d, range);
         TR = d.TR.ptr;
     }
     PoissonArgs<T> a;
@@ -936,8 +943,9 @@ template <class T> void Operator::launch_poisson_device(T const* x, T* y, T* TR,
     a.PK = d.PK.ptr;
     a.PF = reinterpret_cast<int2 const*>(d.PF.ptr);
     a.num_elements = int64_t(E_);
-    TDG_HIP(launch_poisson_mfma<T>(int(D_), int(N_), a, x, y, TR, ncols, ncols > 1 ? ld : 0,
-                                   int64_t(trace_entries()), stream_));
+    for (int c0 = 0; c0 < ncols; c0 += range)
+        TDG_HIP(launch_poisson_mfma<T>(int(D_), int(N_), a, x + c0 * ld, y + c0 * ld, TR, std::min(range, ncols - c0),
+                                       ncols > 1 ? ld : 0, int64_t(trace_entries()), stream_));
 }
 
 template <class T> static std::vector<T> cast(std::vector<double> const& v) {

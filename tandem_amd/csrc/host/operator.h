@@ -280,6 +280,7 @@ private:
     template <class T> void upload_poisson(DevicePoisson<T>& d);
     template <class T> void reserve_poisson(DevicePoisson<T>& d, int ncols);
     template <class T> void launch_poisson_device(T const* x, T* y, T* TR, int ncols, int64_t ld);
+    int poisson_columns(int pb, int ncols) const;
     std::size_t trace_entries() const { return E_ * (D_ + 1) * nq_ * 2; }
     template <class T> int64_t apply_dot_impl(T const* x, T* y, double* partials);
     void ensure_mfma_faces();

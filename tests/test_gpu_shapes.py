@@ -179,3 +179,19 @@ def test_multigrid_few_columns(cuda, D, n, degrees, fp32):
             op.apply(X[c, :op.n].contiguous(), y)
             assert torch.equal(y, Y[c, :op.n])
         assert torch.all(Y[:, op.n:] == 7.0)
+
+
+def test_poisson_column_ranges(cuda):
+    """More columns than one range of the Poisson trace buffer (1 GiB) holds: every column as singly."""
+    import torch
+
+    c = Mixed(3, (7, 7, 7), 4, kind=1, seed=2)
+    one = c.op.E * 4 * c.op.nq * 2 * 8
+    cols = (1 << 30) // one + 3
+    X = torch.rand((cols, c.n), dtype=torch.float64, device=cuda)
+    Y = torch.full_like(X, float("nan"))
+    c.op.apply_batched(X, Y)
+    for k in (0, cols - 4, cols - 3, cols - 1):
+        y = torch.empty(c.n, dtype=torch.float64, device=cuda)
+        c.op.apply(X[k].contiguous(), y)
+        assert torch.equal(y, Y[k])
