@@ -30,10 +30,14 @@
 
 namespace tdg {
 
+// (the runtime's last error is cleared with the throw: the next launch checks its own)
 #define TDG_HIP(call)                                                                              \
     do {                                                                                           \
         hipError_t e_ = (call);                                                                    \
-        if (e_ != hipSuccess) throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e_)); \
+        if (e_ != hipSuccess) {                                                                    \
+            (void)hipGetLastError();                                                               \
+            throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e_));          \
+        }                                                                                          \
     } while (0)
 
 template <class T> void DeviceArray<T>::reset() {
@@ -488,6 +492,7 @@ void Operator::reserve_columns(int ncols) {
 template <class T> void Operator::reserve_split(DeviceSplit<T>& ds, int ncols) {
     if (ds.cap >= ncols) return;
     const std::size_t per = E_ * (D_ + 1) * block_size();
+    ds.cap = 0; // the old slots are gone if the allocation fails
     ds.L.alloc(per * std::size_t(ncols));
     TDG_HIP(hipMemsetAsync(ds.L.ptr, 0, ds.L.n * sizeof(T), stream_));
     TDG_HIP(hipStreamSynchronize(stream_));
@@ -864,6 +869,7 @@ template <class T> DevicePoisson<T>& Operator::device_poisson() {
 
 template <class T> void Operator::reserve_poisson(DevicePoisson<T>& d, int ncols) {
     if (d.cap >= ncols) return;
+    d.cap = 0; // the old traces are gone if the allocation fails
     d.TR.alloc(trace_entries() * std::size_t(ncols));
     d.cap = ncols;
 }

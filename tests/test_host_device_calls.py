@@ -1,0 +1,87 @@
+"""What the library asks of the HIP runtime, in order (no GPU: a runtime of host memory answers and logs
+the calls, kernels do not run): allocations and the buffers the launches write, streams, launch choices.
+Each scenario runs in a process of its own, where that runtime is loaded before the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, re, sys
+F = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+F.fake_log.restype, F.fake_log.argtypes = C.c_size_t, [C.c_char_p, C.c_size_t]
+F.fake_limit.argtypes, F.fake_capture.argtypes = [C.c_size_t], [C.c_void_p]
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import tandem_amd as T
+from tandem_amd._lib import lib
+
+def log(pattern=""):
+    b = C.create_string_buffer(F.fake_log(None, 0))
+    F.fake_log(b, len(b))
+    F.fake_clear()
+    return [l for l in b.value.decode().splitlines() if re.search(pattern, l)]
+
+def operator(kind, D, n, N):
+    op = T.DGOperator(T.Mesh.box(D, n, 1 if D == 3 else 0, 5), kind, N)
+    one = np.ones((op.E, op.Nq))
+    op.set_material(one, one if kind == 0 else None)
+    return op
+
+X, Y = C.c_void_p(1 << 20), C.c_void_p(1 << 21)  # vectors that no host code touches
+MULT = {8: lib().tdg_mult, 4: lib().tdg_mult_f32}
+BATCH = {8: lib().tdg_mult_batched, 4: lib().tdg_mult_batched_f32}
+
+def traces(lines):
+    return {l.split()[-1] for l in lines if "poisson_trace" in l or "poisson_element" in l}
+"""
+
+
+@pytest.fixture(scope="session")
+def host_hip(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "host_hip.so")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I/opt/rocm/include",
+                           os.path.join(HERE, "fake_hip.cpp"), "-o", so])
+
+    def run(code):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + code, so, ROOT], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+
+    return run
+
+
+def test_batch_that_finds_no_memory_leaves_single_applies_whole(host_hip):
+    """A column count whose facet slots do not fit is an error; the one-column apply after it allocates its
+    slots again instead of writing through the lost buffer."""
+    host_hip("""
+op = operator(0, 3, 2, 4)
+for pb in (8, 4):
+    assert MULT[pb](op._h, X, Y) == 0
+    F.fake_limit(1 << 22)
+    assert BATCH[pb](op._h, X, Y, 64, op.n) == -3 and b"out of memory" in lib().tdg_last_error()
+    F.fake_limit(1 << 40)
+    log()
+    assert MULT[pb](op._h, X, Y) == 0
+    assert any(int(l.split()[2]) == op.n * 4 * pb for l in log("^malloc")), "slots of one column"
+""")
+
+
+def test_poisson_batch_that_finds_no_memory_leaves_single_applies_whole(host_hip):
+    """The same for the traces of the matrix-core Poisson apply: no launch writes a buffer that is gone."""
+    host_hip("""
+op = operator(1, 3, 14, 1)
+for pb in (8, 4):
+    assert MULT[pb](op._h, X, Y) == 0
+    F.fake_limit(1 << 22)
+    BATCH[pb](op._h, X, Y, 64, op.n)
+    F.fake_limit(1 << 40)
+    log()
+    assert MULT[pb](op._h, X, Y) == 0
+    used = traces(log())
+    assert used and "(nil)" not in used
+""")
