@@ -485,8 +485,8 @@ void Operator::reserve_columns(int ncols) {
         reserve_split(*s64_, ncols);
         reserve_split(*s32_, ncols);
     }
-    if (uses_poisson_mfma(8, ncols)) reserve_poisson(device_poisson<double>(), poisson_columns(8, ncols));
-    if (uses_poisson_mfma(4, ncols)) reserve_poisson(device_poisson<float>(), poisson_columns(4, ncols));
+    if (int n = ncols; uses_poisson_mfma(8, ncols)) poisson_traces(device_poisson<double>(), n);
+    if (int n = ncols; uses_poisson_mfma(4, ncols)) poisson_traces(device_poisson<float>(), n);
 }
 
 template <class T> void Operator::reserve_split(DeviceSplit<T>& ds, int ncols) {
@@ -848,10 +848,10 @@ bool Operator::uses_poisson_mfma(int pb, int ncols) const {
     return kernel_rule_sizes(D_, N_, &kq, &kf) == 0 && kq == int(Nq_) && kf == int(nq_);
 }
 
-// Columns a matrix-core Poisson apply takes at a time: its traces (about four vectors a column) stay within
-// 1 GiB, or one column's.
-int Operator::poisson_columns(int pb, int ncols) const {
-    return int(std::max<int64_t>(1, std::min<int64_t>(ncols, (int64_t(1) << 30) / int64_t(trace_entries() * pb))));
+// Columns a matrix-core Poisson apply takes at a time at most: their traces (about four vectors a column)
+// stay within 256 MiB, or one column's.
+int Operator::poisson_columns(int pb) const {
+    return int(std::max<int64_t>(1, std::min<int64_t>(65535, (int64_t(1) << 28) / int64_t(trace_entries() * pb))));
 }
 
 template <class T> DevicePoisson<T>& Operator::device_poisson() {
@@ -867,11 +867,20 @@ template <class T> DevicePoisson<T>& Operator::device_poisson() {
     return *slot;
 }
 
-template <class T> void Operator::reserve_poisson(DevicePoisson<T>& d, int ncols) {
-    if (d.cap >= ncols) return;
-    d.cap = 0; // the old traces are gone if the allocation fails
-    d.TR.alloc(trace_entries() * std::size_t(ncols));
-    d.cap = ncols;
+// The trace buffer of an apply of ncols columns; ncols becomes the columns that it holds, if fewer.  Buffers
+// of several columns at least double, so that they hold less than twice the limit together.
+template <class T> T* Operator::poisson_traces(DevicePoisson<T>& d, int& ncols) {
+    const int most = poisson_columns(int(sizeof(T)));
+    ncols = std::min(ncols, most);
+    if (ncols <= 1) return d.TR.ptr;
+    if (ncols > d.cap) {
+        const int cap = std::min(most, std::max(ncols, 2 * d.cap));
+        auto b = std::make_unique<DeviceArray<T>>();
+        b->alloc(trace_entries() * std::size_t(cap));
+        d.batch.push_back(std::move(b));
+        d.cap = cap;
+    }
+    return d.batch.back()->ptr;
 }
 
 // Point data of the matrix-core Poisson apply in groups of 16 elements, element innermost (layouts and
@@ -930,17 +939,13 @@ template <class T> void Operator::upload_poisson(DevicePoisson<T>& d) {
     d.PV.upload(PV);
     d.PK.upload(PK);
     d.PF.upload(PF);
-    d.cap = 0;
-    reserve_poisson(d, 1);
+    d.TR.alloc(trace_entries());
 }
 
 template <class T> void Operator::launch_poisson_device(T const* x, T* y, T* TR, int ncols, int64_t ld) {
     DevicePoisson<T>& d = device_poisson<T>();
-    const int range = poisson_columns(int(sizeof(T)), ncols);
-    if (!TR) {
-        reserve_poisson(d, range);
-        TR = d.TR.ptr;
-    }
+    int range = ncols;
+    if (!TR) TR = poisson_traces(d, range);
     PoissonArgs<T> a;
     a.V = d.V.ptr;
     a.F = d.F.ptr;

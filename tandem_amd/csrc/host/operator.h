@@ -68,10 +68,13 @@ template <class T> struct DeviceSplit {
 };
 
 // Tables and element-grouped point data of the matrix-core Poisson apply (PoissonArgs), and the traces
-// of its two kernels (cap columns).
+// of its two kernels: one buffer for single columns and, from the first batch on, buffers for several, of
+// which the last (cap columns) is used.  A buffer stays where it is for the life of this object: a
+// captured apply replays into the one that it was captured with.
 template <class T> struct DevicePoisson {
     DeviceArray<T> V, F, w, PV, PK, TR;
     DeviceArray<int32_t> PF; // int2 per element face
+    std::vector<std::unique_ptr<DeviceArray<T>>> batch;
     int cap = 0;
 };
 
@@ -278,9 +281,9 @@ private:
     bool uses_poisson_mfma(int pb, int ncols) const;
     template <class T> DevicePoisson<T>& device_poisson();
     template <class T> void upload_poisson(DevicePoisson<T>& d);
-    template <class T> void reserve_poisson(DevicePoisson<T>& d, int ncols);
+    template <class T> T* poisson_traces(DevicePoisson<T>& d, int& ncols);
     template <class T> void launch_poisson_device(T const* x, T* y, T* TR, int ncols, int64_t ld);
-    int poisson_columns(int pb, int ncols) const;
+    int poisson_columns(int pb) const;
     std::size_t trace_entries() const { return E_ * (D_ + 1) * nq_ * 2; }
     template <class T> int64_t apply_dot_impl(T const* x, T* y, double* partials);
     void ensure_mfma_faces();

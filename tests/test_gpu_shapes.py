@@ -182,7 +182,7 @@ def test_multigrid_few_columns(cuda, D, n, degrees, fp32):
 
 
 def test_poisson_column_ranges(cuda):
-    """More columns than one range of the Poisson trace buffer (1 GiB) holds: every column as singly."""
+    """More columns than four ranges of the Poisson trace buffer (256 MiB) hold: every column as singly."""
     import torch
 
     c = Mixed(3, (7, 7, 7), 4, kind=1, seed=2)

@@ -85,3 +85,32 @@ for pb in (8, 4):
     used = traces(log())
     assert used and "(nil)" not in used
 """)
+
+
+@pytest.mark.parametrize("pb", [8, 4])
+def test_poisson_traces_stay_in_place(host_hip, pb):
+    """No apply frees a trace buffer that an earlier one was launched with (a captured apply replays into
+    it), and all of them together stay bounded whatever column counts come."""
+    host_hip("""
+pb = %d
+op = operator(1, 3, 14, 1)
+op.upload()
+log()
+one = op.E * 4 * op.nq * 2 * pb
+seen = []
+for cols in (1, 2, 7, 64, 3, 300, 1, 1000):
+    assert (MULT[pb](op._h, X, Y) if cols == 1 else BATCH[pb](op._h, X, Y, cols, op.n)) == 0
+    lines = log()
+    seen += [int(l.split()[2]) for l in lines if l.startswith("malloc")]
+    assert not [l for l in lines if l.startswith("free")], cols
+    used = traces(lines)
+    assert len(used) == 1
+    if cols == 1:
+        single = single if cols > 1 or "single" in globals() else used
+        assert used == single
+    # columns a launch takes fit the buffer that it writes
+    assert sum(int(l.split("x")[1].split()[0]) for l in lines if "poisson_trace" in l) == cols
+assert sum(seen) <= 2 * (1 << 28) and max(seen) > (1 << 28) - one
+op.set_material(np.ones((op.E, op.Nq)))  # a new material gives everything back
+assert len(log("^free")) >= len(seen)
+""" % pb)
