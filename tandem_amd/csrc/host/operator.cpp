@@ -40,6 +40,19 @@ namespace tdg {
         }                                                                                          \
     } while (0)
 
+// Device memory that is not there (the same message and status code as any other HIP error).
+struct OutOfDeviceMemory : std::runtime_error {
+    OutOfDeviceMemory() : std::runtime_error(std::string("HIP error: ") + hipGetErrorString(hipErrorOutOfMemory)) {}
+};
+
+// Whether work on stream s is being captured rather than run (the default stream cannot be captured).
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!s || hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
 template <class T> void DeviceArray<T>::reset() {
     if (ptr) (void)hipFree(ptr);
     ptr = nullptr;
@@ -48,7 +61,13 @@ template <class T> void DeviceArray<T>::reset() {
 template <class T> void DeviceArray<T>::alloc(std::size_t count) {
     reset();
     if (count == 0) return;
-    TDG_HIP(hipMalloc(reinterpret_cast<void**>(&ptr), count * sizeof(T)));
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&ptr), count * sizeof(T));
+    if (e != hipSuccess) ptr = nullptr;
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        throw OutOfDeviceMemory();
+    }
+    TDG_HIP(e);
     n = count;
 }
 template <class T> void DeviceArray<T>::upload(std::vector<T> const& h) {
@@ -411,6 +430,7 @@ void Operator::drop_device() {
     s32_.reset();
     p64_.reset();
     p32_.reset();
+    p_none_[0] = p_none_[1] = false;
     rhs64_.reset();
     bj_.reset();
     asm_.reset();
@@ -485,8 +505,8 @@ void Operator::reserve_columns(int ncols) {
         reserve_split(*s64_, ncols);
         reserve_split(*s32_, ncols);
     }
-    if (int n = ncols; uses_poisson_mfma(8, ncols)) poisson_traces(device_poisson<double>(), n);
-    if (int n = ncols; uses_poisson_mfma(4, ncols)) poisson_traces(device_poisson<float>(), n);
+    if (uses_poisson_mfma(8, ncols)) poisson_traces<double>(ncols);
+    if (uses_poisson_mfma(4, ncols)) poisson_traces<float>(ncols);
 }
 
 template <class T> void Operator::reserve_split(DeviceSplit<T>& ds, int ncols) {
@@ -854,33 +874,47 @@ int Operator::poisson_columns(int pb) const {
     return int(std::max<int64_t>(1, std::min<int64_t>(65535, (int64_t(1) << 28) / int64_t(trace_entries() * pb))));
 }
 
-template <class T> DevicePoisson<T>& Operator::device_poisson() {
+// The data of the matrix-core Poisson apply, built on first use; null where the device has no memory for them
+// (until the next upload) or a capture is under way: such applies run the thread-per-point kernel, which needs
+// nothing but the operator.
+template <class T> DevicePoisson<T>* Operator::device_poisson() {
     auto& slot = [&]() -> auto& {
         if constexpr (std::is_same<T, double>::value) return p64_;
         else return p32_;
     }();
-    if (!slot) {
-        auto d = std::make_unique<DevicePoisson<T>>();
-        upload_poisson(*d);
-        slot = std::move(d);
+    bool& none = p_none_[sizeof(T) == 8 ? 0 : 1];
+    if (!slot && !none && !capturing(stream_)) {
+        try {
+            auto d = std::make_unique<DevicePoisson<T>>();
+            upload_poisson(*d);
+            slot = std::move(d);
+        } catch (OutOfDeviceMemory const&) {
+            none = true;
+        }
     }
-    return *slot;
+    return slot.get();
 }
 
-// The trace buffer of an apply of ncols columns; ncols becomes the columns that it holds, if fewer.  Buffers
-// of several columns at least double, so that they hold less than twice the limit together.
-template <class T> T* Operator::poisson_traces(DevicePoisson<T>& d, int& ncols) {
-    const int most = poisson_columns(int(sizeof(T)));
-    ncols = std::min(ncols, most);
-    if (ncols <= 1) return d.TR.ptr;
-    if (ncols > d.cap) {
-        const int cap = std::min(most, std::max(ncols, 2 * d.cap));
+// The trace buffer of an apply of ncols columns and the columns that it takes at a time (0: no matrix-core
+// apply now).  Buffers of several columns at least double, so that they hold less than twice the limit
+// together; where a larger one cannot be had (no memory, or a capture is under way) the apply goes through
+// the one there is.
+template <class T> std::pair<T*, int> Operator::poisson_traces(int ncols) {
+    DevicePoisson<T>* const d = device_poisson<T>();
+    if (!d) return {nullptr, 0};
+    const int most = poisson_columns(int(sizeof(T))), want = std::min(ncols, most);
+    if (want > 1 && want > d->cap && !capturing(stream_)) {
+        const int cap = std::min(most, std::max(want, 2 * d->cap));
         auto b = std::make_unique<DeviceArray<T>>();
-        b->alloc(trace_entries() * std::size_t(cap));
-        d.batch.push_back(std::move(b));
-        d.cap = cap;
+        try {
+            b->alloc(trace_entries() * std::size_t(cap));
+            d->batch.push_back(std::move(b));
+            d->cap = cap;
+        } catch (OutOfDeviceMemory const&) {
+        }
     }
-    return d.batch.back()->ptr;
+    if (want > 1 && d->cap > 0) return {d->batch.back()->ptr, std::min(want, d->cap)};
+    return {d->TR.ptr, 1};
 }
 
 // Point data of the matrix-core Poisson apply in groups of 16 elements, element innermost (layouts and
@@ -942,10 +976,9 @@ template <class T> void Operator::upload_poisson(DevicePoisson<T>& d) {
     d.TR.alloc(trace_entries());
 }
 
-template <class T> void Operator::launch_poisson_device(T const* x, T* y, T* TR, int ncols, int64_t ld) {
-    DevicePoisson<T>& d = device_poisson<T>();
-    int range = ncols;
-    if (!TR) TR = poisson_traces(d, range);
+// Ranges of columns through the traces TR, `range` at a time.
+template <class T>
+void Operator::launch_poisson_device(DevicePoisson<T> const& d, T const* x, T* y, T* TR, int range, int ncols, int64_t ld) {
     PoissonArgs<T> a;
     a.V = d.V.ptr;
     a.F = d.F.ptr;
@@ -957,6 +990,16 @@ template <class T> void Operator::launch_poisson_device(T const* x, T* y, T* TR,
     for (int c0 = 0; c0 < ncols; c0 += range)
         TDG_HIP(launch_poisson_mfma<T>(int(D_), int(N_), a, x + c0 * ld, y + c0 * ld, TR, std::min(range, ncols - c0),
                                        ncols > 1 ? ld : 0, int64_t(trace_entries()), stream_));
+}
+
+// The matrix-core apply, if its data and traces are there for ranges that it is the faster choice for; else
+// nothing is done and the caller runs the thread-per-point kernel.
+template <class T> bool Operator::try_poisson_mfma(T const* x, T* y, int ncols, int64_t ld) {
+    if (!uses_poisson_mfma(int(sizeof(T)), ncols)) return false;
+    const auto [TR, range] = poisson_traces<T>(ncols);
+    if (range == 0 || (range < ncols && !uses_poisson_mfma(int(sizeof(T)), range))) return false;
+    launch_poisson_device(*device_poisson<T>(), x, y, TR, range, ncols, ld);
+    return true;
 }
 
 template <class T> static std::vector<T> cast(std::vector<double> const& v) {
@@ -1743,9 +1786,7 @@ template <class T> void Operator::dispatch(T const* x, T* y, int ncols, int64_t 
     } else if (uses_mfma()) {
         if constexpr (std::is_same<T, double>::value) launch_mfma(*m64_, x, y, ncols, ld);
         else launch_mfma(*m32_, x, y, ncols, ld);
-    } else if (uses_poisson_mfma(int(sizeof(T)), ncols)) {
-        launch_poisson_device<T>(x, y, nullptr, ncols, ld);
-    } else {
+    } else if (!try_poisson_mfma<T>(x, y, ncols, ld)) {
         launch(device<T>(), x, y, ncols, ld);
     }
 }
@@ -1814,7 +1855,7 @@ void Operator::apply_noalloc(double const* x, double* y, double* scratch, std::s
     if (uses_poisson_mfma(8, 1)) {
         // the traces go to the scratch memory; operators whose traces it cannot hold, or that were uploaded for
         // another variant, take the kernel without any
-        if (p64_ && trace_entries() <= cap) launch_poisson_device<double>(x, y, scratch, 1, 0);
+        if (p64_ && trace_entries() <= cap) launch_poisson_device<double>(*p64_, x, y, scratch, 1, 1, 0);
         else launch(*d64_, x, y, 1, 0);
         return;
     }

@@ -13,6 +13,7 @@
 #include <functional>
 #include <memory>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace tdg {
@@ -279,10 +280,12 @@ private:
     template <class T> void reserve_split(DeviceSplit<T>& s, int ncols);
     // whether an apply of ncols columns in pb bytes a real takes the matrix-core Poisson kernels
     bool uses_poisson_mfma(int pb, int ncols) const;
-    template <class T> DevicePoisson<T>& device_poisson();
+    template <class T> DevicePoisson<T>* device_poisson();
     template <class T> void upload_poisson(DevicePoisson<T>& d);
-    template <class T> T* poisson_traces(DevicePoisson<T>& d, int& ncols);
-    template <class T> void launch_poisson_device(T const* x, T* y, T* TR, int ncols, int64_t ld);
+    template <class T> std::pair<T*, int> poisson_traces(int ncols);
+    template <class T>
+    void launch_poisson_device(DevicePoisson<T> const& d, T const* x, T* y, T* TR, int range, int ncols, int64_t ld);
+    template <class T> bool try_poisson_mfma(T const* x, T* y, int ncols, int64_t ld);
     int poisson_columns(int pb) const;
     std::size_t trace_entries() const { return E_ * (D_ + 1) * nq_ * 2; }
     template <class T> int64_t apply_dot_impl(T const* x, T* y, double* partials);
@@ -332,6 +335,7 @@ private:
     std::unique_ptr<DeviceSplit<float>> s32_;
     std::unique_ptr<DevicePoisson<double>> p64_;
     std::unique_ptr<DevicePoisson<float>> p32_;
+    bool p_none_[2] = {false, false}; // FP64 / FP32: no device memory for them in this upload
     std::unique_ptr<DeviceRhs> rhs64_;
     std::unique_ptr<BlockJacobi> bj_;
     std::unique_ptr<DeviceAssembled> asm_;

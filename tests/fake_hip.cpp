@@ -17,7 +17,7 @@ namespace {
 std::vector<std::string> g_log;
 std::map<void const*, std::string> g_names;
 std::map<void*, size_t> g_live;
-size_t g_limit = size_t(1) << 40;
+size_t g_total = 0, g_limit = size_t(1) << 40;
 hipStream_t g_capturing = nullptr;
 hipError_t g_last = hipSuccess;
 double g_clock = 0.0;
@@ -39,7 +39,7 @@ hipError_t fail(hipError_t e) { return g_last = e; }
 extern "C" {
 // controls
 void fake_clear() { g_log.clear(); }
-void fake_limit(size_t bytes) { g_limit = bytes; }           // larger allocations find no memory
+void fake_room(size_t bytes) { g_limit = g_total + bytes; } // device memory left
 void fake_capture(void* s) { g_capturing = hipStream_t(s); } // the stream under capture
 size_t fake_log(char* out, size_t n) {
     std::string s;
@@ -50,17 +50,18 @@ size_t fake_log(char* out, size_t n) {
 
 hipError_t hipMalloc(void** p, size_t n) {
     if (g_capturing) return fail(hipErrorStreamCaptureUnsupported);
-    if (n > g_limit) {
+    if (g_total + n > g_limit) {
         log("nomem %zu", n);
         return fail(hipErrorOutOfMemory);
     }
     *p = std::calloc(n, 1);
-    g_live[*p] = n;
+    g_total += g_live[*p] = n;
     log("malloc %p %zu", *p, n);
     return hipSuccess;
 }
 hipError_t hipFree(void* p) {
     log("free %p", p);
+    g_total -= g_live[p];
     g_live.erase(p);
     std::free(p);
     return hipSuccess;

@@ -14,7 +14,7 @@ PRELUDE = """
 import ctypes as C, re, sys
 F = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 F.fake_log.restype, F.fake_log.argtypes = C.c_size_t, [C.c_char_p, C.c_size_t]
-F.fake_limit.argtypes, F.fake_capture.argtypes = [C.c_size_t], [C.c_void_p]
+F.fake_room.argtypes, F.fake_capture.argtypes = [C.c_size_t], [C.c_void_p]
 sys.path.insert(0, sys.argv[2])
 import numpy as np
 import tandem_amd as T
@@ -62,9 +62,9 @@ def test_batch_that_finds_no_memory_leaves_single_applies_whole(host_hip):
 op = operator(0, 3, 2, 4)
 for pb in (8, 4):
     assert MULT[pb](op._h, X, Y) == 0
-    F.fake_limit(1 << 22)
+    F.fake_room(1 << 22)
     assert BATCH[pb](op._h, X, Y, 64, op.n) == -3 and b"out of memory" in lib().tdg_last_error()
-    F.fake_limit(1 << 40)
+    F.fake_room(1 << 40)
     log()
     assert MULT[pb](op._h, X, Y) == 0
     assert any(int(l.split()[2]) == op.n * 4 * pb for l in log("^malloc")), "slots of one column"
@@ -77,9 +77,9 @@ def test_poisson_batch_that_finds_no_memory_leaves_single_applies_whole(host_hip
 op = operator(1, 3, 14, 1)
 for pb in (8, 4):
     assert MULT[pb](op._h, X, Y) == 0
-    F.fake_limit(1 << 22)
+    F.fake_room(1 << 22)
     BATCH[pb](op._h, X, Y, 64, op.n)
-    F.fake_limit(1 << 40)
+    F.fake_room(1 << 40)
     log()
     assert MULT[pb](op._h, X, Y) == 0
     used = traces(log())
@@ -113,4 +113,55 @@ for cols in (1, 2, 7, 64, 3, 300, 1, 1000):
 assert sum(seen) <= 2 * (1 << 28) and max(seen) > (1 << 28) - one
 op.set_material(np.ones((op.E, op.Nq)))  # a new material gives everything back
 assert len(log("^free")) >= len(seen)
+""" % pb)
+
+
+@pytest.mark.parametrize("pb", [8, 4])
+def test_poisson_apply_under_capture_needs_nothing_new(host_hip, pb):
+    """What could be captured before the operator had any traces still can: after the upload every column
+    count, and variants switched in between, by the kernels whose data are there."""
+    host_hip("""
+pb = %d
+S = 1 << 12
+for n, cols in ((14, 1), (14, 64), (5, 64)):      # large, and of a size that only batches take the rule
+    for reserved in (False, True):
+        op = operator(1, 3, n, 1)
+        if not reserved:
+            lib().tdg_set_variant(op._h, 1)       # uploaded for another variant
+        op.upload()
+        lib().tdg_set_variant(op._h, 0)
+        if reserved:
+            assert BATCH[pb](op._h, X, Y, cols, op.n) == 0
+        assert lib().tdg_set_stream(op._h, C.c_void_p(S)) == 0
+        F.fake_capture(S)
+        log()
+        assert BATCH[pb](op._h, X, Y, cols, op.n) == 0, (n, cols, reserved, lib().tdg_last_error())
+        F.fake_capture(None)
+        lines = log("launch")
+        assert bool(traces(lines)) == reserved and len(lines) >= 1 and all("stream 0x1000 " in l for l in lines)
+""" % pb)
+
+
+@pytest.mark.parametrize("pb", [8, 4])
+def test_poisson_operator_without_memory_for_traces(host_hip, pb):
+    """An operator that fits the device without the matrix-core apply's data still works, on the kernel that
+    needs none; without memory for a batch's traces the batch goes through those there are."""
+    host_hip("""
+pb = %d
+op = operator(1, 3, 14, 1)
+lib().tdg_set_variant(op._h, 1)
+op.upload()
+lib().tdg_set_variant(op._h, 0)
+F.fake_room(op.n * pb * 3)      # the traces of one column are four vectors and more
+assert MULT[pb](op._h, X, Y) == 0, lib().tdg_last_error()
+assert log("launch") and not log("poisson_trace")
+F.fake_room(1 << 40)
+op.set_material(np.ones((op.E, op.Nq)))
+assert MULT[pb](op._h, X, Y) == 0
+one = traces(log())
+assert one
+F.fake_room(op.E * 4 * op.nq * 2 * pb + 1)
+assert BATCH[pb](op._h, X, Y, 3, op.n) == 0
+lines = log("launch")
+assert traces(lines) == one and len(lines) == 6
 """ % pb)
