@@ -92,11 +92,11 @@ int tdg_mult_f32(tdg_op* op, float const* x, float* y);
  * reference.  The facet slots of the two-kernel apply live in a fixed 64 MiB device array of the
  * library (each GPU holds it until the process ends): operators whose slots need more
  * (elements x (dim+1) x block size doubles > 2^23, about 20,000 P4 tetrahedra) are rejected with
- * TDG_ERR_ARG.  Poisson operators large enough for the matrix-core apply keep its traces there where they
- * fit and otherwise run the kernel that needs none.  The operator must be on the device already (tdg_upload, which also sets up the array
+ * TDG_ERR_ARG.  The operator must be on the device already (tdg_upload, which also sets up the array
  * on the current device, or one tdg_mult), else TDG_ERR_STATE; with TDG_VARIANT_ASSEMBLED it must
- * have been assembled (tdg_assemble or one tdg_mult), and the apply then uses no scratch memory.  All calls on one GPU share the
- * array: calls that overlap in time on one GPU race; calls ordered on one stream do not. */
+ * have been assembled (tdg_assemble or one tdg_mult).  All calls of the two-kernel apply on one GPU share the
+ * array: such calls that overlap in time on one GPU race; calls ordered on one stream do not.  Assembled
+ * and Poisson operators do not use it. */
 int tdg_mult_noalloc(tdg_op* op, double const* x, double* y);
 /* Y(:, c) = A X(:, c) for ncols columns with leading dimension ld (>= local size). */
 int tdg_mult_batched(tdg_op* op, double const* X, double* Y, int ncols, int64_t ld);

@@ -1852,10 +1852,8 @@ void Operator::apply_noalloc(double const* x, double* y, double* scratch, std::s
     if (!have)
         throw std::logic_error("the allocation-free apply needs the operator on the device: call tdg_upload "
                                "(or one tdg_mult) first");
-    if (uses_poisson_mfma(8, 1)) {
-        // the traces go to the scratch memory; operators whose traces it cannot hold, or that were uploaded for
-        // another variant, take the kernel without any
-        if (p64_ && trace_entries() <= cap) launch_poisson_device<double>(*p64_, x, y, scratch, 1, 1, 0);
+    if (kind_ == Kind_Poisson) { // the operator's own traces, or the kernel without any; no scratch memory
+        if (p64_ && uses_poisson_mfma(8, 1)) launch_poisson_device<double>(*p64_, x, y, p64_->TR.ptr, 1, 1, 0);
         else launch(*d64_, x, y, 1, 0);
         return;
     }

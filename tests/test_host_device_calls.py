@@ -165,3 +165,22 @@ assert BATCH[pb](op._h, X, Y, 3, op.n) == 0
 lines = log("launch")
 assert traces(lines) == one and len(lines) == 6
 """ % pb)
+
+
+def test_poisson_noalloc_applies_share_nothing(host_hip):
+    """tdg_mult_noalloc of two Poisson operators: neither writes memory of the other (they may overlap in
+    time on two streams), whatever their size, and nothing is allocated."""
+    host_hip("""
+used = []
+for n in (14, 20):
+    op = operator(1, 3, n, 1)
+    op.upload()
+    globals()["op%d" % n] = op
+    log()
+    assert lib().tdg_mult_noalloc(op._h, X, Y) == 0
+    lines = log()
+    assert not [l for l in lines if l.startswith("malloc")]
+    used.append(traces(lines))
+    assert MULT[8](op._h, X, Y) == 0 and traces(log()) == used[-1]
+assert used[0] and used[1] and not used[0] & used[1]
+""")
