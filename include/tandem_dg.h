@@ -102,7 +102,10 @@ int tdg_mult_noalloc(tdg_op* op, double const* x, double* y);
 int tdg_mult_batched(tdg_op* op, double const* X, double* Y, int ncols, int64_t ld);
 int tdg_mult_batched_f32(tdg_op* op, float const* X, float* Y, int ncols, int64_t ld);
 
-/* Stream all device work of this operator is queued on (hipStream_t; NULL = default stream). */
+/* Stream all device work of this operator is queued on (hipStream_t; NULL = default stream).  The operator's
+ * work buffers (facet slots, Poisson traces) serve one apply after another: the new stream waits for the
+ * work queued on the old one, unless one of them is under capture.  A graph of captured applies uses the
+ * same buffers; launch it where it does not overlap other applies of the operator. */
 int tdg_set_stream(tdg_op* op, void* stream);
 
 /* Kernel choice: TDG_VARIANT_AUTO (default) runs the two-kernel matrix-core (MFMA) apply where one

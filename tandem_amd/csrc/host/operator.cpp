@@ -45,12 +45,13 @@ struct OutOfDeviceMemory : std::runtime_error {
     OutOfDeviceMemory() : std::runtime_error(std::string("HIP error: ") + hipGetErrorString(hipErrorOutOfMemory)) {}
 };
 
-// Whether work on stream s is being captured rather than run (the default stream cannot be captured).
+// Whether work on stream s is being captured rather than run, or a capture elsewhere forbids it to run (the
+// default stream, while a blocking stream is captured), or the stream is gone.
 static bool capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (!s || hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
     (void)hipGetLastError();
-    return false;
+    return true;
 }
 
 template <class T> void DeviceArray<T>::reset() {
@@ -107,7 +108,9 @@ Operator::Operator(SimplexMesh mesh, int kind, unsigned degree, std::vector<doub
     build_geometry(geometry_nodes);
 }
 
-Operator::~Operator() = default;
+Operator::~Operator() {
+    if (handover_) (void)hipEventDestroy(handover_);
+}
 
 void Operator::build_tables() {
     unsigned order = 2 * N_ + 1; // MinQuadOrder() (app/config.h.in:8-11)
@@ -517,6 +520,19 @@ template <class T> void Operator::reserve_split(DeviceSplit<T>& ds, int ncols) {
     TDG_HIP(hipMemsetAsync(ds.L.ptr, 0, ds.L.n * sizeof(T), stream_));
     TDG_HIP(hipStreamSynchronize(stream_));
     ds.cap = ncols;
+}
+
+// The old stream's work and the new stream's meet in the operator's buffers (facet slots, traces, the wave
+// and fault work vectors), so the new stream waits for the old one.  An operator without any, and streams
+// under capture (what they record runs when the caller launches the graph), are left alone.
+void Operator::set_stream(hipStream_t s) {
+    const bool shared = s64_ || s32_ || p64_ || p32_ || wave_ || fault_;
+    if (s != stream_ && shared && !capturing(s) && !capturing(stream_)) {
+        if (!handover_) TDG_HIP(hipEventCreateWithFlags(&handover_, hipEventDisableTiming));
+        TDG_HIP(hipEventRecord(handover_, stream_));
+        TDG_HIP(hipStreamWaitEvent(s, handover_, 0));
+    }
+    stream_ = s;
 }
 
 void Operator::set_variant(int v) {

@@ -166,7 +166,9 @@ public:
     void upload_device();
     template <class T> DeviceOperator<T> const& device();
 
-    void set_stream(hipStream_t s) { stream_ = s; }
+    // Later work goes to stream s, after the work already queued on the old stream: both use the operator's
+    // work buffers.
+    void set_stream(hipStream_t s);
     hipStream_t stream() const { return stream_; }
     void set_variant(int v);
     int variant() const { return variant_; }
@@ -305,6 +307,7 @@ private:
     QuadRule vol_, fct_;
     bool ready_ = false;
     hipStream_t stream_ = nullptr;
+    hipEvent_t handover_ = nullptr; // orders a new stream after the old one
 
     // reference tables (FP64)
     std::vector<double> E_Q_, Dxi_Q_;                       // solution basis at volume points

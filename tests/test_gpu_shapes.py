@@ -195,3 +195,43 @@ def test_poisson_column_ranges(cuda):
         y = torch.empty(c.n, dtype=torch.float64, device=cuda)
         c.op.apply(X[k].contiguous(), y)
         assert torch.equal(y, Y[k])
+
+
+@pytest.mark.parametrize("D,n,N", [(2, (65, 63), 4), (3, (11, 10, 10), 2)])
+def test_poisson_captured_and_on_two_streams(cuda, D, n, N):
+    """The matrix-core Poisson apply captured into a graph and replayed after a larger batch, with eager
+    applies between, and applies of two vectors queued on two streams in turn: the eager results' bits."""
+    import torch
+
+    c = Mixed(D, n, N, kind=1, seed=3)
+    c.op.upload()
+    X = torch.rand((5, c.n), dtype=torch.float64, device=cuda)
+    ref = torch.empty_like(X)
+    for k in range(5):
+        c.op.apply(X[k], ref[k])
+    x, y, Y = X[0].clone(), torch.zeros_like(X[0]), torch.empty_like(X)
+    s, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=s):
+        c.op.set_stream(s)
+        c.op.apply(x, y)
+    c.op.set_stream(None)
+    c.op.apply_batched(X, Y)
+    assert torch.equal(Y, ref)
+    for k in (1, 4, 2):
+        x.copy_(X[k])
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        c.op.apply(X[k - 1], Y[0])
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref[k]) and torch.equal(Y[0], ref[k - 1])
+    Y.fill_(float("nan"))
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for i in range(40):
+        c.op.set_stream(streams[i % 2])
+        c.op.apply(X[i % 5], Y[i % 5])
+    c.op.set_stream(None)
+    torch.cuda.synchronize()
+    assert torch.equal(Y, ref)

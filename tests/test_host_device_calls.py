@@ -184,3 +184,31 @@ for n in (14, 20):
     assert MULT[8](op._h, X, Y) == 0 and traces(log()) == used[-1]
 assert used[0] and used[1] and not used[0] & used[1]
 """)
+
+
+@pytest.mark.parametrize("kind,N,n,shared", [(1, 1, 14, True), (0, 2, 2, True), (1, 1, 3, False)])
+def test_new_stream_waits_for_the_old_one(host_hip, kind, N, n, shared):
+    """Applies queued on one stream and then on another meet in the operator's buffers: the new stream waits
+    for the old one; not under capture, nor where an operator has no such buffers."""
+    host_hip("""
+op = operator(%d, 3, %d, %d)
+shared = %s
+A, B = 1 << 12, 1 << 13
+def streams(s):
+    log()
+    assert lib().tdg_set_stream(op._h, C.c_void_p(s)) == 0
+    return log("record|wait")
+assert streams(A) == []                       # nothing on the device yet
+op.upload()
+assert MULT[8](op._h, X, Y) == 0
+lines = streams(B)
+if shared:
+    (r, rs, re_), (w, ws, we) = [l.split() for l in lines]
+    assert (r, rs, w, ws) == ("record", hex(A), "wait", hex(B)) and re_ == we
+else:
+    assert lines == []
+assert streams(B) == []                       # the same stream again
+assert len(streams(None)) == len(lines)
+F.fake_capture(A)
+assert streams(A) == [] and MULT[8](op._h, X, Y) == 0 and streams(B) == []
+""" % (kind, n, N, shared))
