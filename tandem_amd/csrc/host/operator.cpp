@@ -1619,6 +1619,7 @@ void Operator::assembled_host(std::vector<double>& A, std::vector<int32_t>& nb) 
 }
 
 template <class T> AssembledArgs<T> Operator::assembled_args() const {
+    if (!asm_) throw std::logic_error("the operator has not been assembled");
     AssembledArgs<T> a{};
     if constexpr (std::is_same<T, double>::value) a.A = asm_->A64.ptr;
     else a.A = asm_->A32.ptr;

@@ -60,7 +60,8 @@ private:
     template <class T>
     void step(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* out, int64_t ldo, int ncols, int k);
     template <class T>
-    void residual(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* r, int64_t ldr, int ncols);
+    void residual(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* r, int64_t ldr, int ncols,
+                  bool rows = false);
     template <class T> void cycle(int l, T const* b, int64_t ldb, T* x, int64_t ldx, int ncols);
 
     Operator& op_;

@@ -775,12 +775,12 @@ void AMG::step(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* out, 
     }
 }
 
-// r = b - A_l x
+// r = b - A_l x; rows (level 0): by the few-column kernel of the block rows
 template <class T>
-void AMG::residual(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* r, int64_t ldr, int ncols) {
+void AMG::residual(int l, T const* b, int64_t ldb, T const* x, int64_t ldx, T* r, int64_t ldr, int ncols, bool rows) {
     AMGLevelDev& v = *lv_[l];
     hipStream_t st = op_.stream();
-    if (l == 0 && ncols <= kFewColumns) {
+    if (l == 0 && rows) {
         AssembledStep<T> p;
         p.b = b;
         p.x = x;
@@ -849,14 +849,16 @@ template <class T> void AMG::cycle(int l, T const* b, int64_t ldb, T* x, int64_t
     AMGLevelDev& c = *lv_[l + 1];
     LevelVectors<T>& w = v.w<T>();
     LevelVectors<T>& wc = c.w<T>();
-    if (ncols <= kFewColumns) {
+    // (level 0 only while its operator applies by its block rows: a caller may have set another variant, or
+    // a new material that drops the rows until the next such apply)
+    if (ncols <= kFewColumns && (l > 0 || (op_.variant() == Variant_Assembled && op_.assembled()))) {
         // every step is one launch that reads the neighbours' old x and writes the other vector
         T *u[2] = {w.z.p, w.t.p}, *cur = nullptr;
         for (int k = 0; k < o_.smooth; ++k) {
             step<T>(l, b, ldb, cur, v.ld, u[k & 1], v.ld, ncols, k);
             cur = u[k & 1];
         }
-        residual<T>(l, b, ldb, cur, v.ld, w.r.p, v.ld, ncols);
+        residual<T>(l, b, ldb, cur, v.ld, w.r.p, v.ld, ncols, true);
         bsr_launch<0>(v.R, static_cast<T const*>(w.r.p), v.ld, wc.b.p, c.ld, static_cast<T const*>(nullptr), 0, ncols,
                       st);
         cycle<T>(l + 1, wc.b.p, c.ld, wc.x.p, c.ld, ncols);

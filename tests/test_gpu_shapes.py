@@ -235,3 +235,24 @@ def test_poisson_captured_and_on_two_streams(cuda, D, n, N):
     c.op.set_stream(None)
     torch.cuda.synchronize()
     assert torch.equal(Y, ref)
+
+
+def test_multigrid_coarse_operator_changed_after_setup(cuda):
+    """A coarse operator that a caller has given another variant, and a new material besides (its block rows
+    are dropped), still serves one and two columns: the set-up's AMG levels precondition what it now applies."""
+    import torch
+
+    cs = [Mixed(3, (4, 3, 5), N, seed=9) for N in (2, 1)]
+    fine, coarse = cs
+    B = torch.from_numpy(np.random.default_rng(13).uniform(-1.0, 1.0, (2, fine.n))).to(cuda)
+    mg = T.PMultigrid([c.op for c in cs], galerkin_penalty=0)
+    assert mg.solve_multi(B, torch.zeros_like(B), rtol=1e-10)["converged"]
+    for change in (lambda: coarse.op.set_variant("auto"), lambda: coarse.op.set_material(*coarse.c),
+                   lambda: coarse.op.set_variant("assembled")):
+        change()
+        for k in (1, 2):
+            X = torch.zeros_like(B)
+            assert mg.solve_multi(B[:k].contiguous(), X[:k], rtol=1e-10)["converged"]
+            for c in range(k):
+                r = B[c].cpu().numpy() - fine.oracle.apply(X[c].cpu().numpy())
+                assert np.linalg.norm(r) <= 1e-9 * float(torch.linalg.norm(B[c]))
