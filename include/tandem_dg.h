@@ -149,9 +149,12 @@ int tdg_autotune(tdg_op* op, int ncols, int precision_bytes, int* chosen, double
  * on ncols columns in FP64 (precision_bytes 8) or FP32 (4), keeps the fastest for that precision,
  * reports it in *shape and *xcd and the milliseconds per apply in ms[TDG_SPLIT_ORDERS shape + xcd]
  * (TDG_SPLIT_ORDERS x TDG_SPLIT_SHAPES entries, -1 if the operator has no two-kernel apply).  tdg_set_shape selects one directly.
- * Until a shape is selected, applies of few elements (up to 1024 groups of 16 elements times columns, or
- * 384 groups of 8 facets) run with launches made for them, whose waves share each group; the search keeps
- * those for such operators where they are the faster choice.  tdg_autotune runs the shape search before it compares the variants.  No counterpart in the reference (its kernels are
+ * Until a shape is selected with tdg_set_shape, applies of few elements (up to 1024 groups of 16 elements times
+ * columns, or 384 groups of 8 facets) run with launches made for them, whose waves share each group, instead
+ * of the shape.  The search leaves that so; where its shape is faster than they are on the ncols that it
+ * timed, applies of that many columns take the shape.  A column's result depends in its last bits on the
+ * kernels taken, hence on the number of columns applied with it where that number decides between them.
+ * tdg_autotune runs the shape search before it compares the variants.  No counterpart in the reference (its kernels are
  * generated for one CPU target). */
 enum { TDG_SPLIT_SHAPES = 4, TDG_SPLIT_ORDERS = 3 };
 int tdg_autotune_shapes(tdg_op* op, int ncols, int precision_bytes, int* shape, int* xcd, double* ms);

@@ -605,38 +605,42 @@ std::vector<double> Operator::autotune_shapes(int ncols, int pb) {
     if (!(kind_ == Kind_Elasticity && mfma_supported(D_, N_)))
         return std::vector<double>(kSplitOrders * kSplitShapes, -1.0);
     const int saved_variant = variant_, saved_shape = split_shape_[p], saved_xcd = split_xcd_[p];
+    const int saved_off = split_off_cols_[p];
     const bool saved_auto = split_auto_[p];
-    // the last configuration: the default shape with the small launches, where the rule takes any
-    const int last = kSplitOrders * kSplitShapes;
-    bool small = false;
     try {
         variant_ = Variant_Auto;
-        time_configs(ncols, pb, last + 1, [&](int c) {
-            split_auto_[p] = c == last;
-            split_shape_[p] = c == last ? saved_shape : c / kSplitOrders;
-            split_xcd_[p] = c == last ? saved_xcd : c % kSplitOrders;
-            if (c == last) small = split_small_bits(pb, ncols) != 0;
-            return c < last || small;
+        split_auto_[p] = false;
+        time_configs(ncols, pb, kSplitOrders * kSplitShapes, [&](int c) {
+            split_shape_[p] = c / kSplitOrders;
+            split_xcd_[p] = c % kSplitOrders;
+            return true;
         }, ms);
+        int best = 0;
+        for (int c = 1; c < kSplitOrders * kSplitShapes; ++c)
+            if (ms[std::size_t(c)] < ms[std::size_t(best)]) best = c;
+        split_shape_[p] = best / kSplitOrders;
+        split_xcd_[p] = best % kSplitOrders;
+        // the small launches, where the rule takes any for this column count, against that shape: where they
+        // lose, this count does without them; other counts follow the rule
+        split_auto_[p] = true;
+        split_off_cols_[p] = 0;
+        if (split_small_bits(pb, ncols) != 0) {
+            std::vector<double> two;
+            time_configs(ncols, pb, 2, [&](int c) {
+                split_off_cols_[p] = c == 0 ? ncols : 0;
+                return true;
+            }, two);
+            split_off_cols_[p] = two[0] <= two[1] ? ncols : 0;
+        }
     } catch (...) {
         variant_ = saved_variant;
         split_shape_[p] = saved_shape;
         split_xcd_[p] = saved_xcd;
+        split_off_cols_[p] = saved_off;
         split_auto_[p] = saved_auto;
         throw;
     }
     variant_ = saved_variant;
-    int best = 0;
-    for (int c = 1; c < last; ++c)
-        if (ms[std::size_t(c)] >= 0.0 && ms[std::size_t(c)] < ms[std::size_t(best)]) best = c;
-    split_shape_[p] = best / kSplitOrders;
-    split_xcd_[p] = best % kSplitOrders;
-    split_auto_[p] = small && ms[std::size_t(last)] < ms[std::size_t(best)];
-    if (split_auto_[p]) {
-        split_shape_[p] = saved_shape;
-        split_xcd_[p] = saved_xcd;
-    }
-    ms.resize(std::size_t(last));
     return ms;
 }
 
@@ -682,7 +686,8 @@ void Operator::set_split_shape(int pb, int shape, int xcd) {
 
 // Which kernels of a two-kernel apply of ncols columns take their small launch.
 int Operator::split_small_bits(int pb, int ncols) const {
-    if (!split_auto_[pb == 8 ? 0 : 1]) return 0;
+    const int p = pb == 8 ? 0 : 1;
+    if (!split_auto_[p] || ncols == split_off_cols_[p]) return 0;
     const int64_t facets = pb == 8 ? (s64_ ? s64_->nfacets : 0) : (s32_ ? s32_->nfacets : 0);
     return split_small(pb, int(Nq_), (facets + 7) / 8 * ncols, int64_t((E_ + 15) / 16) * ncols);
 }

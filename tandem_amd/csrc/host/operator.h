@@ -177,7 +177,8 @@ public:
     // variant (negative where a variant does not apply).
     std::vector<double> autotune(int ncols, int precision_bytes);
     // Launch shapes of the two-kernel apply: times shape s with workgroup order x (0 linear, 1 one
-    // contiguous range per XCD) at index 2 s + x, keeps the fastest for that precision.
+    // contiguous range per XCD, 2 the same, persistent) at index kSplitOrders s + x, keeps the fastest for that
+    // precision, and beside it the small launches for the column counts whose rule takes them.
     std::vector<double> autotune_shapes(int ncols, int precision_bytes);
     void set_split_shape(int precision_bytes, int shape, int xcd);
     int split_shape(int precision_bytes) const { return split_shape_[precision_bytes == 8 ? 0 : 1]; }
@@ -356,8 +357,10 @@ private:
     // 24^3-cube P4 workload; the autotuner re-chooses per operator)
     int split_shape_[2] = {0, 1};
     int split_xcd_[2] = {2, 1};
-    // whether small applies take the shape made for them instead (until a shape is chosen explicitly)
+    // whether small applies take the launches made for them instead (until a shape is chosen explicitly), and
+    // the column count, if any, for which a search found them slower than its shape
     bool split_auto_[2] = {true, true};
+    int split_off_cols_[2] = {0, 0};
     int split_small_bits(int pb, int ncols) const;
     double time_configs(int ncols, int pb, int count, std::function<bool(int)> const& select, std::vector<double>& ms);
 };

@@ -20,7 +20,7 @@ std::map<void*, size_t> g_live;
 size_t g_total = 0, g_limit = size_t(1) << 40;
 hipStream_t g_capturing = nullptr;
 hipError_t g_last = hipSuccess;
-double g_clock = 0.0;
+double g_clock = 1e6, g_step = 1.0;
 struct Call {
     dim3 grid, block;
     size_t shared;
@@ -41,6 +41,7 @@ extern "C" {
 void fake_clear() { g_log.clear(); }
 void fake_room(size_t bytes) { g_limit = g_total + bytes; } // device memory left
 void fake_capture(void* s) { g_capturing = hipStream_t(s); } // the stream under capture
+void fake_step(double ms) { g_step = ms; } // every timed interval is this much longer than the one before
 size_t fake_log(char* out, size_t n) {
     std::string s;
     for (auto const& l : g_log) s += l + "\n";
@@ -102,9 +103,9 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { // every interval longer than the last
-    *ms = float(g_clock += 1.0);
-    log("elapsed %g", g_clock);
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+    *ms = float(g_clock += g_step);
+    log("elapsed %.0f", g_clock);
     return hipSuccess;
 }
 hipError_t hipGetDevice(int* d) {

@@ -15,6 +15,7 @@ import ctypes as C, re, sys
 F = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 F.fake_log.restype, F.fake_log.argtypes = C.c_size_t, [C.c_char_p, C.c_size_t]
 F.fake_room.argtypes, F.fake_capture.argtypes = [C.c_size_t], [C.c_void_p]
+F.fake_step.argtypes = [C.c_double]
 sys.path.insert(0, sys.argv[2])
 import numpy as np
 import tandem_amd as T
@@ -212,3 +213,35 @@ assert len(streams(None)) == len(lines)
 F.fake_capture(A)
 assert streams(A) == [] and MULT[8](op._h, X, Y) == 0 and streams(B) == []
 """ % (kind, n, N, shared))
+
+
+@pytest.mark.parametrize("precision,pb", [("fp64", 8), ("fp32", 4)])
+def test_shape_search_leaves_the_small_launches(host_hip, precision, pb):
+    """A shape searched for many columns governs the launches that the rule for few elements leaves to it: a
+    one-column apply of the same mesh keeps its small launches (a facet group a workgroup of five waves), and a
+    count for which they were the slower choice does without them."""
+    host_hip("""
+precision, pb = "%s", %d
+op = operator(0, 3, 4, 4)
+def small(cols):
+    log()
+    assert (MULT[pb](op._h, X, Y) if cols == 1 else BATCH[pb](op._h, X, Y, cols, op.n)) == 0
+    (f,) = log("facet_kernel")
+    return " block 320 " in f
+assert small(1) and small(2) and not small(64)
+for step in (1.0, -1.0):
+    F.fake_step(step)
+    shape, ms = op.autotune_shapes(64, precision)
+    assert small(1) and small(2) and not small(64)
+    assert ms[shape] == min(ms.values())
+F.fake_step(1.0)                    # the later a configuration is timed, the slower it is
+shape, ms = op.autotune_shapes(1, precision)
+assert ms[shape] == min(ms.values()) and not small(1) and small(2)
+F.fake_step(-1.0)
+shape, ms = op.autotune_shapes(1, precision)
+assert ms[shape] == min(ms.values()) and small(1) and small(2)
+op.set_shape(precision, *shape)     # chosen by the caller: for every apply
+assert not small(1) and not small(2)
+F.fake_step(1.0)
+assert op.autotune(64, precision)[0] == "auto" and small(1)
+""" % (precision, pb))
