@@ -245,3 +245,24 @@ assert not small(1) and not small(2)
 F.fake_step(1.0)
 assert op.autotune(64, precision)[0] == "auto" and small(1)
 """ % (precision, pb))
+
+
+@pytest.mark.parametrize("precision,order", [("fp64", 2), ("fp64", 0), ("fp32", 1)])
+def test_shape_search_for_columns_leaves_the_order(host_hip, precision, order):
+    """Several columns take the same launch in every workgroup order: noise between equal launches does not
+    choose the order of single applies."""
+    host_hip("""
+precision, order = "%s", %d
+op = operator(0, 3, 4, 4)
+op.set_shape(precision, 1, order)
+for step in (1.0, -1.0, 1.0):
+    F.fake_step(step)
+    log()
+    shape, ms = op.autotune_shapes(64, precision)
+    assert shape[1] == order and shape[0] == (0 if step > 0 else 3)
+    assert len(log("elapsed")) == 2 * 4
+    assert len(ms) == 12 and all(ms[s, o] == ms[s, order] for s, o in ms)
+    assert ms[shape] == min(ms.values())
+F.fake_step(1.0)
+assert op.autotune_shapes(1, precision)[0] == (0, 0)   # a single column times every order
+""" % (precision, order))
