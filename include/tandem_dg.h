@@ -134,7 +134,8 @@ int tdg_set_variant(tdg_op* op, int variant);
 
 /* Autotuner: times every variant that applies to the operator (the two-kernel MFMA apply, the
  * element-centric MFMA kernel with linear and XCD-grouped workgroup order, the thread-per-point
- * kernel) on ncols columns in FP64 (precision_bytes 8) or FP32 (4), keeps the fastest as the
+ * kernel, the assembled register kernel; for Poisson above its size rule the matrix-core apply, below it
+ * TDG_VARIANT_AUTO is the thread-per-point kernel and is kept in its place) on ncols columns in FP64 (precision_bytes 8) or FP32 (4), keeps the fastest as the
  * operator's variant and reports it in *chosen and the milliseconds per apply in ms[variant]
  * (TDG_NUM_VARIANTS entries, -1 where a variant does not apply).  No counterpart in the
  * reference (its kernels are generated for one CPU target). */

@@ -678,6 +678,12 @@ std::vector<double> Operator::autotune(int ncols, int pb) {
     int best = -1;
     for (int v = 0; v < kNumVariants; ++v)
         if (ms[std::size_t(v)] >= 0.0 && (best < 0 || ms[std::size_t(v)] < ms[std::size_t(best)])) best = v;
+    // Poisson below its size rule: the automatic choice is the thread-per-point kernel at this column count and
+    // the matrix-core apply at larger ones, so where that kernel wins the choice stays open
+    if (poisson_mfma_compiled() && ms[Variant_Auto] < 0.0) {
+        ms[Variant_Auto] = ms[Variant_Points];
+        if (best == Variant_Points) best = Variant_Auto;
+    }
     variant_ = best;
     return ms;
 }
@@ -887,12 +893,15 @@ template <class T> void Operator::upload_split(DeviceSplit<T>& ds) {
     reserve_split(ds, 1);
 }
 
-bool Operator::uses_poisson_mfma(int pb, int ncols) const {
-    if (kind_ != Kind_Poisson || variant_ != Variant_Auto ||
-        int64_t(local_size()) * ncols < poisson_mfma_unknowns(int(D_), pb) || (D_ == 2 && N_ == 1))
-        return false;
+bool Operator::poisson_mfma_compiled() const {
     int kq = 0, kf = 0;
-    return kernel_rule_sizes(D_, N_, &kq, &kf) == 0 && kq == int(Nq_) && kf == int(nq_);
+    return kind_ == Kind_Poisson && !(D_ == 2 && N_ == 1) && kernel_rule_sizes(D_, N_, &kq, &kf) == 0 &&
+           kq == int(Nq_) && kf == int(nq_);
+}
+
+bool Operator::uses_poisson_mfma(int pb, int ncols) const {
+    return kind_ == Kind_Poisson && variant_ == Variant_Auto &&
+           int64_t(local_size()) * ncols >= poisson_mfma_unknowns(int(D_), pb) && poisson_mfma_compiled();
 }
 
 // Columns a matrix-core Poisson apply takes at a time at most: their traces (about four vectors a column)

@@ -281,7 +281,9 @@ private:
     template <class T> void upload_split(DeviceSplit<T>& d);
     template <class T> SplitArgs<T> split_args(DeviceMfma<T> const& m, DeviceSplit<T> const& s) const;
     template <class T> void reserve_split(DeviceSplit<T>& s, int ncols);
-    // whether an apply of ncols columns in pb bytes a real takes the matrix-core Poisson kernels
+    // whether an apply of ncols columns in pb bytes a real takes the matrix-core Poisson kernels (by size; by
+    // operator: whether they are compiled for it)
+    bool poisson_mfma_compiled() const;
     bool uses_poisson_mfma(int pb, int ncols) const;
     template <class T> DevicePoisson<T>* device_poisson();
     template <class T> void upload_poisson(DevicePoisson<T>& d);

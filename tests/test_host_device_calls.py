@@ -266,3 +266,29 @@ for step in (1.0, -1.0, 1.0):
 F.fake_step(1.0)
 assert op.autotune_shapes(1, precision)[0] == (0, 0)   # a single column times every order
 """ % (precision, order))
+
+
+def test_poisson_search_below_the_size_rule_leaves_the_choice_open(host_hip):
+    """Tuned at a size where the automatic choice and "points" are the same kernel, a Poisson operator still
+    takes the matrix-core apply for more columns; a faster assembled apply, or a choice at a size where both
+    kernels ran, is kept."""
+    host_hip("""
+op = operator(1, 3, 5, 2)          # 7,500 unknowns; no assembled register kernel
+for precision, pb in (("fp64", 8), ("fp32", 4)):
+    name, ms = op.autotune(1, precision)
+    assert name == "auto" and ms["auto"] == ms["points"]
+    log()
+    assert MULT[pb](op._h, X, Y) == 0 and not traces(log())
+    assert BATCH[pb](op._h, X, Y, 64, op.n) == 0 and traces(log())
+    F.fake_step(-1.0)
+    assert op.autotune(1, precision)[0] == "auto"
+    assert op.autotune(64, precision)[0] == "points"
+    F.fake_step(1.0)
+    assert op.autotune(64, precision)[0] == "auto"
+small = operator(1, 3, 5, 1)       # block size 4: the assembled register kernel
+F.fake_step(-1.0)
+assert small.autotune(1, "fp64")[0] == "assembled"
+F.fake_step(1.0)
+assert small.autotune(1, "fp64")[0] == "auto"
+assert operator(1, 2, 5, 1).autotune(1, "fp64")[0] == "points"   # no matrix-core apply at any size
+""")
