@@ -171,7 +171,7 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
     using vec = T __attribute__((ext_vector_type(VW), aligned(sizeof(T))));
 
     __shared__ T sT[NF * nq * NbfP];
-    __shared__ int sP[2 * NF * Nbf];
+    __shared__ int sP[NF * Nbf]; // face-frame label -> element node
     __shared__ T sW[nq];
     __shared__ T sX[W][16 * BSP];
 
@@ -179,9 +179,9 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
     {
         const int tid = threadIdx.x;
 #pragma unroll
-        for (int i0 = 0; i0 < 2 * NF * Nbf; i0 += 64 * W) {
+        for (int i0 = 0; i0 < NF * Nbf; i0 += 64 * W) {
             const int i = i0 + tid;
-            if (i < 2 * NF * Nbf) sP[i] = a.perm[i];
+            if (i < NF * Nbf) sP[i] = a.perm[i];
         }
 #pragma unroll
         for (int i0 = 0; i0 < nT; i0 += 64 * W) {

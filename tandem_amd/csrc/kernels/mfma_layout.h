@@ -89,7 +89,7 @@ hipError_t launch_elasticity_mfma(int dim, int degree, MfmaArgs<T> const& a, T c
 template <class T> struct SplitArgs {
     T const* V;
     T const* T0;
-    int32_t const* perm; // [2][f][k] face-frame label -> element node, then its inverse
+    int32_t const* perm; // [f][k] face-frame label -> element node
     T const* w;
     T const* VD;
     T const* FR;
