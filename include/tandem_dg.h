@@ -149,9 +149,9 @@ int tdg_autotune(tdg_op* op, int ncols, int precision_bytes, int* chosen, double
  * workgroups as are resident, each looping over its blocks).  tdg_autotune_shapes times all of them
  * on ncols columns in FP64 (precision_bytes 8) or FP32 (4), keeps the fastest for that precision,
  * reports it in *shape and *xcd and the milliseconds per apply in ms[TDG_SPLIT_ORDERS shape + xcd]
- * (TDG_SPLIT_ORDERS x TDG_SPLIT_SHAPES entries, -1 if the operator has no two-kernel apply).  Several columns
- * go through one launch whatever the order: each shape is timed once then, reported for its three orders,
- * and the order stays.  tdg_set_shape selects one directly.
+ * (TDG_SPLIT_ORDERS x TDG_SPLIT_SHAPES entries, -1 if the operator has no two-kernel apply).  For several
+ * columns orders 0 and 1 are one launch: it is timed once and reported for both, and of the two the search
+ * keeps the one that is set (1 if 2 is).  tdg_set_shape selects one directly.
  * Until a shape is selected with tdg_set_shape, applies of few elements (up to 1024 groups of 16 elements times
  * columns, or 384 groups of 8 facets) run with launches made for them, whose waves share each group, instead
  * of the shape.  The search leaves that so; where its shape is faster than they are on the ncols that it

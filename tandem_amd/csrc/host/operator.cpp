@@ -610,20 +610,21 @@ std::vector<double> Operator::autotune_shapes(int ncols, int pb) {
     try {
         variant_ = Variant_Auto;
         split_auto_[p] = false;
-        // several columns: the workgroups take a block's columns in turn and the orders are one launch (two where
-        // a workgroup takes all columns), so only the order set is timed, and it stays for the single applies
-        const int order = ncols > 1 ? saved_xcd : -1;
+        // several columns: the linear and the per-XCD order are one launch (a block's columns follow each other
+        // on one XCD), timed once
+        const bool cols = ncols > 1;
         time_configs(ncols, pb, kSplitOrders * kSplitShapes, [&](int c) {
             split_shape_[p] = c / kSplitOrders;
             split_xcd_[p] = c % kSplitOrders;
-            return order < 0 || split_xcd_[p] == order;
+            return !(cols && split_xcd_[p] == 1);
         }, ms);
-        int best = std::max(order, 0);
+        int best = 0;
         for (int c = 0; c < kSplitOrders * kSplitShapes; ++c) {
-            if (order >= 0) ms[std::size_t(c)] = ms[std::size_t(c / kSplitOrders * kSplitOrders + order)];
+            if (ms[std::size_t(c)] < 0.0) ms[std::size_t(c)] = ms[std::size_t(c - 1)];
             if (ms[std::size_t(c)] < ms[std::size_t(best)]) best = c;
         }
-        if (order >= 0) best = best / kSplitOrders * kSplitOrders + order;
+        // of the two the one that is set, or the better one for the single applies that it governs too
+        if (cols && best % kSplitOrders == 0 && saved_xcd != 0) ++best;
         split_shape_[p] = best / kSplitOrders;
         split_xcd_[p] = best % kSplitOrders;
         // the small launches, where the rule takes any for this column count, against that shape: where they

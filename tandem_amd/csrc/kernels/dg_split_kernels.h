@@ -105,7 +105,7 @@ __device__ __forceinline__ void block_of(unsigned w, unsigned nvb, int ncols, in
     lb = ncols > 1 ? (r / unsigned(ncols)) * 8u + xcd : (xcd_remap ? xcd * (nvb / 8u) + r : w);
 }
 
-// Runs f(virtual block, column, block) over the blocks of this workgroup.  MC (several columns): one
+// Runs f(virtual block, column, block) over the blocks of this workgroup.  MC (several columns, facet kernel): one
 // block for a.cpw consecutive columns, one after another, so that the tables are loaded once and the
 // block's records come from the CU's own cache after the first column.
 template <bool PERSIST, bool MC, class A, class F>
@@ -548,7 +548,7 @@ void elasticity_facet_kernel(SplitArgs<T> a, T const* __restrict__ xs, T* __rest
 // the slots are read at the end; the other waves of the SIMD cover the waits.
 // SPL > 1 (small meshes): SPL consecutive waves share 16 elements, each taking every SPL-th block of
 // points, and sum their results from LDS as they store them.
-template <int D, int N, class T, int W, int OCC, bool DEEP, bool VTAIL_ON, bool PERSIST, int SPL = 1, bool MC = false>
+template <int D, int N, class T, int W, int OCC, bool DEEP, bool VTAIL_ON, bool PERSIST, int SPL = 1>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(OCC)))
 void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const* __restrict__ Ls,
                                T* __restrict__ ys, int64_t ld, int64_t ldL, int ncols, unsigned nvb) {
@@ -584,7 +584,7 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
     __syncthreads();
 
     auto block = [&](unsigned vb, unsigned col, unsigned lb) {
-        const int tid = int(threadIdx.x), wv = tid >> 6, lane = lane_of<PERSIST || MC>(tid), j = lane & 15, g = lane >> 4;
+        const int tid = int(threadIdx.x), wv = tid >> 6, lane = lane_of<PERSIST>(tid), j = lane & 15, g = lane >> 4;
         T* const U = sU[wv];
         const int part = SPL > 1 ? wv % SPL : 0;
         const int64_t grp = int64_t(lb) * (W / SPL) + wv / SPL;
@@ -873,7 +873,7 @@ void elasticity_element_kernel(SplitArgs<T> a, T const* __restrict__ xs, T const
         }
         wave_sync(); // every read of the staged region is done before the next block restages it
     };
-    for_blocks<PERSIST, MC>(a, ncols, nvb, block);
+    for_blocks<PERSIST, false>(a, ncols, nvb, block);
 }
 
 // Launch shapes of the two kernels, searched by the autotuner: waves per workgroup and the
@@ -923,13 +923,21 @@ hipError_t run_small_elements(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, 
     return hipGetLastError();
 }
 
-// Columns a workgroup takes one after another (its tables loaded once, its records in the CU's cache):
+// Columns a facet workgroup takes one after another (its tables loaded once, its records in the CU's cache):
 // at most 8, fewer where the chip would otherwise get too few workgroups to finish evenly.  us per apply of
-// 64 columns with 1 / 4 / 8 / 16 a visit: 2D P6 FP32 18,432 elements 758 / 720 / 721 / 755, 80,000: 3356 / 3174 /
-// 3117 / 3162; 3D P4 FP64 6,000: 2291 / 2136 / 2427 / 2518, 24,576: 9185 / 8496 / 8308 / 8297.
+// 64 columns without visits, and with 1 / 2 / 4 / 8 / 16 columns each: 2D P6 FP32 18,432 elements 754, 757 / 724 /
+// 728 / 730 / 732, 80,000: 3393, 3427 / 3305 / 3255 / 3210 / 3196; 2D P2 FP64 45,000: 843, 894 / 840 / 809 / 798 / 797;
+// 3D P3 FP32 24,576: 1963, 1969 / 1920 / 1908 / 1905 / 1925.
 inline int columns_per_visit(int64_t blocks, int ncols) {
     return int(std::max<int64_t>(1, std::min<int64_t>({8, ncols, blocks * ncols / 8192})));
 }
+// Whether several columns go by visits: not where the tables are little of a block's work (3D P4 FP64 3,072
+// elements 906, 913 / 923 / 915 / 945 / 1001; FP32 16,464: 2457, 2547 / 2494 / 2465 / 2476 / 2473; 2D P6 FP64 80,000, whose
+// persistent launch loads them once anyway: 6183, 6594 / 6481 / 6360 / 6254 / 6214).  The element kernel never
+// does: the loop over columns takes registers that it has not (3D P4 FP32 spilled 83 of 168 and went from
+// 203 to 398 us at 3,072 elements; without visits 64 columns take 475 us instead of 683, of 16,464 elements
+// 2381 instead of 3293).
+template <int D, int N, class T> constexpr bool facet_visits() { return D == 3 ? N <= 3 : sizeof(T) == 4 || N <= 4; }
 
 template <int D, int N, class T, class S>
 hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols, int64_t ld, int64_t ldL,
@@ -939,19 +947,22 @@ hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols
     const int64_t et = element_workgroups<S>(a.num_groups) * int64_t(ncols);
     if (ft > int64_t(0x7fffffff) || et > int64_t(0x7fffffff)) return hipErrorInvalidValue;
     const bool persist = a.xcd_remap == 2;
+    const int cpw = facet_visits<D, N, T>() && ncols > 1 ? columns_per_visit(ft / ncols, ncols) : 0;
     hipError_t e = hipSuccess;
     if (ft > 0) {
         if (a.small & kSmallFacets) {
             e = a.num_fgroups * ncols <= kSmallOneGroup
                     ? run_small_facets<D, N, T, 1>(a, x, Lbuf, ncols, ld, ldL, s)
                     : run_small_facets<D, N, T, 2>(a, x, Lbuf, ncols, ld, ldL, s);
-        } else if (ncols > 1) {
-            SplitArgs<T> m = a;
-            m.cpw = columns_per_visit(ft / ncols, ncols);
-            const int64_t gf = ft / ncols * ((ncols + m.cpw - 1) / m.cpw);
-            hipLaunchKernelGGL((elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, false, 1, true>),
-                               dim3(unsigned(gf)), dim3(64 * S::fw), 0, s, m, x, Lbuf, ld, ldL, ncols, unsigned(gf));
-            e = hipGetLastError();
+        } else if (cpw > 1 || (cpw == 1 && !persist)) { // (one column a visit: no gain over the persistent launch)
+            if constexpr (facet_visits<D, N, T>()) {
+                SplitArgs<T> m = a;
+                m.cpw = cpw;
+                const int64_t gf = ft / ncols * ((ncols + cpw - 1) / cpw);
+                hipLaunchKernelGGL((elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, false, 1, true>),
+                                   dim3(unsigned(gf)), dim3(64 * S::fw), 0, s, m, x, Lbuf, ld, ldL, ncols, unsigned(gf));
+                e = hipGetLastError();
+            }
         } else if (persist) {
             auto fk = elasticity_facet_kernel<D, N, T, S::fw, S::focc, S::vtail, true>;
             const int64_t fg = resident_workgroups(reinterpret_cast<void const*>(fk), 64 * S::fw, ft);
@@ -969,14 +980,6 @@ hipError_t run_shape(SplitArgs<T> const& a, T const* x, T* y, T* Lbuf, int ncols
         return a.num_groups * ncols <= kSmallOneGroup
                    ? run_small_elements<D, N, T, 1>(a, x, y, Lbuf, ncols, ld, ldL, s)
                    : run_small_elements<D, N, T, 2>(a, x, y, Lbuf, ncols, ld, ldL, s);
-    if (ncols > 1) {
-        SplitArgs<T> m = a;
-        m.cpw = columns_per_visit(et / ncols, ncols);
-        const int64_t ge = et / ncols * ((ncols + m.cpw - 1) / m.cpw);
-        hipLaunchKernelGGL((elasticity_element_kernel<D, N, T, S::ew, S::eocc, S::deep, S::vtail, false, 1, true>),
-                           dim3(unsigned(ge)), dim3(64 * S::ew), 0, s, m, x, Lbuf, y, ld, ldL, ncols, unsigned(ge));
-        return hipGetLastError();
-    }
     if (persist) {
         auto ek = elasticity_element_kernel<D, N, T, S::ew, S::eocc, S::deep, S::vtail, true>;
         const int64_t eg = resident_workgroups(reinterpret_cast<void const*>(ek), 64 * S::ew, et);

@@ -249,23 +249,44 @@ assert op.autotune(64, precision)[0] == "auto" and small(1)
 
 @pytest.mark.parametrize("precision,order", [("fp64", 2), ("fp64", 0), ("fp32", 1)])
 def test_shape_search_for_columns_leaves_the_order(host_hip, precision, order):
-    """Several columns take the same launch in every workgroup order: noise between equal launches does not
-    choose the order of single applies."""
+    """Several columns take the same launch in the linear and the per-XCD order: noise between equal launches
+    does not choose the order of single applies."""
     host_hip("""
 precision, order = "%s", %d
 op = operator(0, 3, 4, 4)
-op.set_shape(precision, 1, order)
-for step in (1.0, -1.0, 1.0):
+for step, kept in ((1.0, 1 if order == 2 else order), (-1.0, 2)):   # the first configuration wins, then the last
+    op.set_shape(precision, 1, order)
     F.fake_step(step)
     log()
     shape, ms = op.autotune_shapes(64, precision)
-    assert shape[1] == order and shape[0] == (0 if step > 0 else 3)
-    assert len(log("elapsed")) == 2 * 4
-    assert len(ms) == 12 and all(ms[s, o] == ms[s, order] for s, o in ms)
+    assert shape == (0 if step > 0 else 3, kept)
+    assert len(log("elapsed")) == 2 * 8
+    assert len(ms) == 12 and all(ms[s, 0] == ms[s, 1] for s in range(4))
     assert ms[shape] == min(ms.values())
 F.fake_step(1.0)
 assert op.autotune_shapes(1, precision)[0] == (0, 0)   # a single column times every order
 """ % (precision, order))
+
+
+@pytest.mark.parametrize("precision,pb", [("fp64", 8), ("fp32", 4)])
+@pytest.mark.parametrize("D,n,N,visits", [(3, 3, 4, False), (3, 5, 2, True), (2, 24, 3, True)])
+def test_kernels_of_several_columns(host_hip, D, n, N, visits, precision, pb):
+    """The element kernel of several columns is the one of single columns (one with a loop over columns has no
+    registers for it), and facet workgroups visit several columns where that pays: every (group, column) once."""
+    host_hip("""
+D, n, N, visits, precision, pb = %r
+op = operator(0, D, n, N)
+for shape in range(4):
+    for order in range(3):
+        op.set_shape(precision, shape, order)
+        log()
+        assert MULT[pb](op._h, X, Y) == 0
+        f1, e1 = log("launch")
+        assert BATCH[pb](op._h, X, Y, 800, op.n) == 0
+        f, e = log("launch")
+        assert "facet" in f and "element" in e and e.split()[1] == e1.split()[1]
+        assert (f.split()[1] != f1.split()[1]) == visits
+""" % ((D, n, N, visits, precision, pb),))
 
 
 def test_poisson_search_below_the_size_rule_leaves_the_choice_open(host_hip):
