@@ -906,9 +906,10 @@ bool Operator::uses_poisson_mfma(int pb, int ncols) const {
 }
 
 // Columns a matrix-core Poisson apply takes at a time at most: their traces (about four vectors a column)
-// stay within 256 MiB, or one column's.
+// stay within 1 GiB, or one column's.  Smaller ranges cost launches (64 columns of 16,464 P4 tetrahedra in FP64:
+// 4460 us, in ranges of 256 MiB 4656).
 int Operator::poisson_columns(int pb) const {
-    return int(std::max<int64_t>(1, std::min<int64_t>(65535, (int64_t(1) << 28) / int64_t(trace_entries() * pb))));
+    return int(std::max<int64_t>(1, std::min<int64_t>(65535, (int64_t(1) << 30) / int64_t(trace_entries() * pb))));
 }
 
 // The data of the matrix-core Poisson apply, built on first use; null where the device has no memory for them

@@ -99,7 +99,7 @@ op.upload()
 log()
 one = op.E * 4 * op.nq * 2 * pb
 seen = []
-for cols in (1, 2, 7, 64, 3, 300, 1, 1000):
+for cols in (1, 2, 7, 64, 3, 300, 1, 3000):
     assert (MULT[pb](op._h, X, Y) if cols == 1 else BATCH[pb](op._h, X, Y, cols, op.n)) == 0
     lines = log()
     seen += [int(l.split()[2]) for l in lines if l.startswith("malloc")]
@@ -111,7 +111,7 @@ for cols in (1, 2, 7, 64, 3, 300, 1, 1000):
         assert used == single
     # columns a launch takes fit the buffer that it writes
     assert sum(int(l.split("x")[1].split()[0]) for l in lines if "poisson_trace" in l) == cols
-assert sum(seen) <= 2 * (1 << 28) and max(seen) > (1 << 28) - one
+assert sum(seen) <= 2 * (1 << 30) and max(seen) > (1 << 30) - one
 op.set_material(np.ones((op.E, op.Nq)))  # a new material gives everything back
 assert len(log("^free")) >= len(seen)
 """ % pb)
