@@ -74,8 +74,8 @@ def test_wave_rhs_degrees(cuda, D, n, N):
 @pytest.mark.parametrize("D,n,N", [(3, (1, 1, 1), 4), (3, (3, 2, 1), 4), (3, (3, 2, 1), 3), (3, (2, 2, 1), 2),
                                    (2, (3, 3), 6), (2, (5, 3), 4), (2, (3, 3), 3)])
 def test_small_apply_and_explicit_shapes(cuda, D, n, N):
-    """The shape of small applies (default here), with the fused dot product of the solvers, and every
-    explicitly chosen launch shape and workgroup order on the same mesh."""
+    """The launches of small applies (default here) and every explicitly chosen launch shape and workgroup
+    order on the same mesh."""
     import torch
 
     c = Mixed(D, n, N, seed=N + 1)
@@ -113,6 +113,26 @@ def test_small_apply_limits(cuda, D, n, N, cols):
     assert res["converged"] and rel_l2(c.oracle.apply(x.cpu().numpy()), ref[0]) <= 1e-7
 
 
+@pytest.mark.parametrize("mode", ["fp64", "fp32-ru"])
+@pytest.mark.parametrize("D,n,N", [(3, (1, 1, 1), 4), (3, (11, 9, 9), 3), (2, (47, 47), 4), (2, (91, 90), 6)])
+def test_fused_dot_of_the_small_launches(cuda, D, n, N, mode):
+    """The solvers' p.Ap from the element kernel's partial sums on the small launches, both precisions: one
+    group of elements a workgroup, two (257 to 1024 groups), and near the upper end of the rule.  A wrong sum
+    gives CG wrong steps; the residual is taken in FP64 by the oracle."""
+    import torch
+
+    c = Mixed(D, n, N, seed=7)
+    groups = (c.op.E + 15) // 16
+    assert groups == 1 or 257 <= groups <= 1024
+    b = c.oracle.apply(np.random.default_rng(15).uniform(-1.0, 1.0, c.n), nthreads=8)
+    bd = torch.from_numpy(b).to(cuda)
+    x = torch.zeros_like(bd)
+    res = c.op.solve(bd, x, rtol=1e-8, mode=mode, precond="block-jacobi", max_iter=20000)  # some 2,700 steps
+    assert res["converged"]
+    r = b - c.oracle.apply(x.cpu().numpy(), nthreads=8)
+    assert np.linalg.norm(r) <= 1e-7 * np.linalg.norm(b)
+
+
 @pytest.mark.parametrize("D,n,N", [(2, (101, 101), 2), (2, (79, 77), 3), (2, (65, 63), 4), (2, (55, 53), 5),
                                    (2, (47, 47), 6), (3, (15, 13, 14), 1), (3, (11, 10, 10), 2), (3, (9, 9, 7), 3),
                                    (3, (7, 7, 7), 4)])
@@ -145,6 +165,7 @@ def test_poisson_matrix_core_apply(cuda, D, n, N):
         c.op.set_variant("points")
         c.op.apply(Xd[1, :c.n].contiguous(), y)
         assert rel_l2(y.double().cpu().numpy(), ref[1]) <= bar
+        assert not torch.equal(y, Y[1, :c.n])  # the other kernel: its sums run in another order
         c.op.set_variant("auto")
 
 
@@ -182,7 +203,7 @@ def test_multigrid_few_columns(cuda, D, n, degrees, fp32):
 
 
 def test_poisson_column_ranges(cuda):
-    """More columns than four ranges of the Poisson trace buffer (256 MiB) hold: every column as singly."""
+    """More columns than one range of the Poisson trace buffer (1 GiB) holds: every column as singly."""
     import torch
 
     c = Mixed(3, (7, 7, 7), 4, kind=1, seed=2)
