@@ -1177,7 +1177,7 @@ RhsArgs Operator::rhs_args() {
             fct[i * 4 + 1] = int32_t(fc.elem[1]);
             fct[i * 4 + 2] = int32_t(fc.local[0]) | (int32_t(fc.local[1]) << 4);
         }
-        std::vector<char> data(E_, 0);
+        std::vector<int32_t> data(E_, 0);
         for (std::size_t i = 0; i < F; ++i)
             if (const int bc = fbc[i] & 0xff; bc == BC_Dirichlet || bc == BC_Fault)
                 data[std::size_t(fct[i * 4])] = data[std::size_t(fct[i * 4 + 1])] = 1;
@@ -1185,6 +1185,7 @@ RhsArgs Operator::rhs_args() {
         for (std::size_t e = 0; e < E_; ++e)
             if (data[e]) elist.push_back(int32_t(e));
         r->elist.upload(elist);
+        r->edata.upload(data);
         r->tabE.upload(tabE);
         r->jw.upload(jw);
         r->fbc.upload(fbc);
@@ -1209,6 +1210,7 @@ RhsArgs Operator::rhs_args() {
     a.fct = reinterpret_cast<int4 const*>(rhs64_->fct.ptr);
     a.tabFt = d.tabFt.ptr;
     a.elist = rhs64_->elist.ptr;
+    a.edata = rhs64_->edata.ptr;
     a.num_elist = int64_t(rhs64_->elist.n);
     a.num_elements = int64_t(E_);
     a.num_facets = int64_t(topo_.facets.size());

@@ -89,7 +89,7 @@ template <class T> struct DeviceGrad {
 struct DeviceRhs {
     DeviceArray<double> tabE, jw;
     DeviceArray<int32_t> fbc, fct; // fct: int4 per facet
-    DeviceArray<int32_t> elist;    // elements with a Dirichlet or Fault face
+    DeviceArray<int32_t> elist, edata; // elements with a Dirichlet or Fault face; whether an element is one
 };
 
 // Data of the elastic-wave kernels: reference inverse mass, basis table, -W/|J| per volume point and a

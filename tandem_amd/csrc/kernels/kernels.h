@@ -136,6 +136,7 @@ struct RhsArgs {
     int4 const* fct;      // [F] element 0, element 1, local face 0 | local face 1 << 4
     double const* tabFt;  // [c][q][k] face-0 facet table, lift order
     int32_t const* elist; // elements with a Dirichlet or Fault face
+    int32_t const* edata; // [E] whether the element is one of them
     int64_t num_elements, num_facets, num_elist;
 };
 

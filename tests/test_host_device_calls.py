@@ -313,3 +313,23 @@ F.fake_step(1.0)
 assert small.autotune(1, "fp64")[0] == "auto"
 assert operator(1, 2, 5, 1).autotune(1, "fp64")[0] == "points"   # no matrix-core apply at any size
 """)
+
+
+def test_right_hand_side_is_one_launch(host_hip):
+    """Volume and facet part of a right-hand side in one launch whatever its data (small calls cost their
+    launches), with a workgroup for every element that has a face with data."""
+    host_hip("""
+for D, n, N in ((3, 2, 1), (2, 9, 4)):
+    op = operator(0, D, n, N)
+    F0, D0 = C.c_void_p(1 << 22), C.c_void_p(1 << 23)
+    grid = {}
+    for force, data in ((F0, D0), (None, D0), (F0, None), (None, None)):
+        log()
+        assert lib().tdg_rhs_device(op._h, force, data, Y, 3, op.E * D * op.Nq, op.F * D * op.nq, op.n) == 0
+        (l,) = log("launch")
+        grid[force is not None, data is not None] = int(l.split("grid ")[1].split("x")[0])
+        assert "x3 " in l
+    f = op.facets()
+    touched = len(set(f[f[:, 4] == 5][:, 0]))
+    assert grid[True, True] == grid[False, True] == grid[True, False] + touched and touched > 0
+""")
