@@ -1347,7 +1347,7 @@ WaveArgs Operator::wave_args() {
                 for (unsigned k = 0; k < n; ++k) M[k + l * n] += vol_.weights[q] * E_Q_[k + n * q] * E_Q_[l + n * q];
         for (unsigned k = 0; k < n; ++k) Minv[k + k * n] = 1.0;
         dense_solve(M, int(n), Minv.data(), int(n));
-        const bool grouped = inverse_mass_grouped(int(D_), int(N_));
+        const bool grouped = inverse_mass_grouped(int(D_), int(N_), int64_t(E_));
         std::vector<double> tab(std::size_t(n) * Nq_, 0.0), w(grouped ? (E_ + 15) / 16 * 16 * Nq_ : E_ * Nq_, 0.0);
         if (grouped) { // P = Mhat^-1 E
             for (unsigned q = 0; q < Nq_; ++q)

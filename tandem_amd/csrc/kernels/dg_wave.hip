@@ -177,10 +177,20 @@ unsigned grid256(int64_t n) { return unsigned(std::min<int64_t>((n + 255) / 256,
 } // namespace
 
 // The degrees whose rule sizes are compiled take the matrix-core kernel; the other operators (3D P5 and
-// P6, for which no apply is compiled) the kernel with run-time sizes.
-bool inverse_mass_grouped(int dim, int degree) { return degree >= 1 && degree <= (dim == 2 ? 6 : 4); }
+// P6, for which no apply is compiled) the kernel with run-time sizes, and so do the smallest 3D P4 meshes, where
+// a workgroup an element is done sooner than a wave's chain through 16 of them (us, run-time sizes and matrix
+// cores: 6 elements 10.2 and 11.3, 162: 10.5 and 12.5, 480: 11.6 and 12.6, 1,296: 21.1 and 12.7; 3D P3 6: 6.7 and 5.6).
+bool inverse_mass_grouped(int dim, int degree, int64_t num_elements) {
+    return degree >= 1 && degree <= (dim == 2 ? 6 : 4) && !(dim == 3 && degree == 4 && num_elements <= 512);
+}
 
 hipError_t launch_inverse_mass(int dim, int degree, WaveArgs const& a, double const* x, double* y, hipStream_t s) {
+    if (!inverse_mass_grouped(dim, degree, a.num_elements)) {
+        const std::size_t shm = std::size_t(a.nbf * a.nquant + a.nq * a.nquant) * sizeof(double);
+        if (shm > 64 * 1024) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(inverse_mass_kernel, dim3(unsigned(a.num_elements)), dim3(kT), shm, s, a, x, y);
+        return hipGetLastError();
+    }
     if (dim == 3) {
         switch (degree) {
         case 1: return run_inverse_mass<3, 1>(a, x, y, s);
@@ -198,10 +208,7 @@ hipError_t launch_inverse_mass(int dim, int degree, WaveArgs const& a, double co
         case 6: return run_inverse_mass<2, 6>(a, x, y, s);
         }
     }
-    const std::size_t shm = std::size_t(a.nbf * a.nquant + a.nq * a.nquant) * sizeof(double);
-    if (shm > 64 * 1024) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(inverse_mass_kernel, dim3(unsigned(a.num_elements)), dim3(kT), shm, s, a, x, y);
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_interpolate(double const* I, int n_to, int n_from, int nquant, int64_t nelem, int transpose,

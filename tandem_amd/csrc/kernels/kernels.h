@@ -63,7 +63,7 @@ struct WaveArgs {
     int nbf, nq, nquant;
     int64_t num_elements;
 };
-bool inverse_mass_grouped(int dim, int degree);
+bool inverse_mass_grouped(int dim, int degree, int64_t num_elements);
 hipError_t launch_inverse_mass(int dim, int degree, WaveArgs const& a, double const* x, double* y, hipStream_t stream);
 // y = I x per element and quantity (I: n_to x n_from row-major), or y = I^T x if transpose.
 hipError_t launch_interpolate(double const* I, int n_to, int n_from, int nquant, int64_t nelem, int transpose,

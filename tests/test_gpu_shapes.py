@@ -51,10 +51,10 @@ def test_face_frame_traces(cuda, D, n, N, variant):
 
 
 @pytest.mark.parametrize("D,n,N", [(3, (3, 1, 1), 1), (3, (1, 1, 1), 3), (2, (3, 3), 1), (2, (3, 5), 2), (2, (4, 2), 4),
-                                   (2, (9, 1), 5), (3, (1, 1, 1), 5)])
+                                   (2, (9, 1), 5), (3, (1, 1, 1), 5), (3, (1, 1, 1), 4), (3, (5, 5, 4), 4)])
 def test_wave_rhs_degrees(cuda, D, n, N):
     """The matrix-core inverse mass at the other degrees and partial groups (3D P5 keeps the kernel with
-    run-time sizes and has no apply), in place too; the facet part added to the elements with data."""
+    run-time sizes and has no apply; 3D P4 takes it up to 512 elements), in place too; the facet part added to the elements with data."""
     import torch
 
     c = Mixed(D, n, N, seed=N)

@@ -333,3 +333,18 @@ for D, n, N in ((3, 2, 1), (2, 9, 4)):
     touched = len(set(f[f[:, 4] == 5][:, 0]))
     assert grid[True, True] == grid[False, True] == grid[True, False] + touched and touched > 0
 """)
+
+
+def test_inverse_mass_of_the_smallest_meshes(host_hip):
+    """3D P4 up to 512 elements and degrees without an apply take a workgroup an element, all else the
+    matrix cores."""
+    host_hip("""
+for D, n, N, mfma in ((3, 1, 4, False), (3, 4, 4, False), (3, 5, 4, True), (3, 1, 3, True), (2, 1, 6, True), (3, 1, 5, False)):
+    op = operator(0, D, n, N)
+    op.upload()
+    log()
+    assert lib().tdg_inverse_mass(op._h, X, Y) == 0
+    (l,) = log("launch")
+    assert ("mfma" in l) == mfma, (D, n, N, l)
+    assert mfma or "grid %dx1" % op.E in l
+""")
