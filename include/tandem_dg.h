@@ -98,7 +98,10 @@ int tdg_mult_f32(tdg_op* op, float const* x, float* y);
  * array: such calls that overlap in time on one GPU race; calls ordered on one stream do not.  Assembled
  * and Poisson operators do not use it. */
 int tdg_mult_noalloc(tdg_op* op, double const* x, double* y);
-/* Y(:, c) = A X(:, c) for ncols columns with leading dimension ld (>= local size). */
+/* Y(:, c) = A X(:, c) for ncols columns with leading dimension ld (>= local size).  A column equals the single
+ * apply bit for bit where the same kernels take both; the small launches (tdg_autotune_shapes) and the Poisson
+ * size rule go by elements x columns, so near those limits they differ in summation order.  Work buffers grow
+ * with the largest column count used. */
 int tdg_mult_batched(tdg_op* op, double const* X, double* Y, int ncols, int64_t ld);
 int tdg_mult_batched_f32(tdg_op* op, float const* X, float* Y, int ncols, int64_t ld);
 
@@ -155,9 +158,7 @@ int tdg_autotune(tdg_op* op, int ncols, int precision_bytes, int* chosen, double
  * Until a shape is selected with tdg_set_shape, applies of few elements (up to 1024 groups of 16 elements times
  * columns, or 384 groups of 8 facets) run with launches made for them, whose waves share each group, instead
  * of the shape.  The search leaves that so; where its shape is faster than they are on the ncols that it
- * timed, applies of that many columns take the shape.  A column's result depends in its last bits on the
- * kernels taken, hence on the number of columns applied with it where that number decides between them.
- * tdg_autotune runs the shape search before it compares the variants.  No counterpart in the reference (its kernels are
+ * timed, applies of that many columns take the shape.  tdg_autotune runs the shape search before it compares the variants.  No counterpart in the reference (its kernels are
  * generated for one CPU target). */
 enum { TDG_SPLIT_SHAPES = 4, TDG_SPLIT_ORDERS = 3 };
 int tdg_autotune_shapes(tdg_op* op, int ncols, int precision_bytes, int* shape, int* xcd, double* ms);

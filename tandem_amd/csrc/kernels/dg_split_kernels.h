@@ -33,7 +33,7 @@
 // every instruction (a quarter of a 64-byte request each), which bound the FP32 kernel (2D P6, 64
 // columns of 18,432 triangles: 620 us in every launch shape, 370 us in pieces; 3D P4 apply 154 -> 133
 // us FP32, 448 -> 433 us FP64).  The vectors are staged as they are; the relabelling is in the offsets
-// of the B operands.  FP64 P4 is then bound by neither roof (matrix cores ~35% busy, ~3 TB/s) but by
+// of the B operands.  FP64 P4 is then bound by neither roof (matrix cores 40% busy, 3.5 TB/s) but by
 // waits at two waves per SIMD.
 //
 // Element kernel.  One wave owns 16 consecutive elements; the volume term is the element-centric

@@ -88,7 +88,10 @@ template <class T>
 hipError_t launch_assembled(AssembledArgs<T> const& a, T const* x, T* y, int ncols, int64_t ld, hipStream_t stream,
                             double* partial = nullptr);
 bool assembled_register_kernel(int block_size, int slots);
-// Few columns (ncols <= kFewColumns): the row kernel (a lane per element row) with a fused epilogue.
+// Few columns (ncols <= kFewColumns): the row kernel (a lane per element row) with a fused epilogue.  (The
+// kernels for few columns are ahead to some 8 columns at 16,464 elements and beyond 16 at 3,072: p-multigrid
+// solves of 3 / 8 / 16 columns with the limit at 2 and at 16: 3,072 elements 319 and 218 / 409 and 303 / 546 and
+// 467 ms; 16,464: 999 and 940 / 1513 and 1464 / 2381 and 2387.  The limit is where they were tried first.)
 //   Residual  out = b - A x
 //   Smooth    z = Dinv (b - A x), d = c1 d + c2 z, out = x + d; x null: the zero guess (out must not be x)
 // Vectors at strides ld (x, out, d) and ldb (b); Dinv[element][bs x bs] column-major.  Block sizes 6 and 12

@@ -417,7 +417,7 @@ __global__ __launch_bounds__(kT) void bsr_wave_kernel(int64_t n, int64_t const* 
 }
 
 // x = Ainv b (dense N x N, row-major), ncols columns: one wave per row (a lane per row left the
-// at most 800 rows on 13 waves that walked a row each: 27 us)
+// at most 800 rows on 13 waves that walked a row each: 27 us; 64 columns 29.0 -> 4.7 us)
 template <class T>
 __global__ __launch_bounds__(kT) void dense_kernel(int64_t N, T const* __restrict__ Ainv, T const* __restrict__ bs,
                                                    int64_t ldb, T* __restrict__ xs, int64_t ldx) {

@@ -221,9 +221,10 @@ class DGOperator:
 
     def set_stream(self, stream):
         """stream: a torch.cuda.Stream (or None for the default stream).  The library's calls are
-        asynchronous on that stream; make it torch's current stream as well (torch.cuda.set_stream
-        or a `with torch.cuda.stream(...)` block), so that the tensors passed in are produced, and
-        their memory recycled by torch's allocator, in the same stream order."""
+        asynchronous on that stream, which first waits for the operator's work on the previous one; make
+        it torch's current stream as well (torch.cuda.set_stream or a `with torch.cuda.stream(...)`
+        block), so that the tensors passed in are produced, and their memory recycled by torch's
+        allocator, in the same stream order."""
         check(lib().tdg_set_stream(self._h, None if stream is None else C.c_void_p(stream.cuda_stream)))
 
     # --- apply
