@@ -505,21 +505,25 @@ void Operator::reserve_columns(int ncols) {
     if (ncols < 1) throw std::invalid_argument("reserve_columns: ncols must be positive");
     upload_device();
     if (uses_split()) {
-        reserve_split(*s64_, ncols);
-        reserve_split(*s32_, ncols);
+        split_slots(*s64_, ncols);
+        split_slots(*s32_, ncols);
     }
     if (uses_poisson_mfma(8, ncols)) poisson_traces<double>(ncols);
     if (uses_poisson_mfma(4, ncols)) poisson_traces<float>(ncols);
 }
 
-template <class T> void Operator::reserve_split(DeviceSplit<T>& ds, int ncols) {
-    if (ds.cap >= ncols) return;
-    const std::size_t per = E_ * (D_ + 1) * block_size();
-    ds.cap = 0; // the old slots are gone if the allocation fails
-    ds.L.alloc(per * std::size_t(ncols));
-    TDG_HIP(hipMemsetAsync(ds.L.ptr, 0, ds.L.n * sizeof(T), stream_));
-    TDG_HIP(hipStreamSynchronize(stream_));
-    ds.cap = ncols;
+// The slots of an apply of ncols columns.
+template <class T> T* Operator::split_slots(DeviceSplit<T>& ds, int ncols) {
+    DeviceArray<T>& L = ncols == 1 ? ds.L : ds.LB;
+    const std::size_t n = E_ * (D_ + 1) * block_size() * std::size_t(ncols);
+    if (ncols == 1 ? !L.ptr : ds.cap < ncols) {
+        if (ncols > 1) ds.cap = 0; // the old slots are gone if the allocation fails
+        L.alloc(n);
+        TDG_HIP(hipMemsetAsync(L.ptr, 0, n * sizeof(T), stream_));
+        TDG_HIP(hipStreamSynchronize(stream_));
+        if (ncols > 1) ds.cap = ncols;
+    }
+    return L.ptr;
 }
 
 // The old stream's work and the new stream's meet in the operator's buffers (facet slots, traces, the wave
@@ -890,8 +894,7 @@ template <class T> void Operator::upload_split(DeviceSplit<T>& ds) {
     ds.idle.upload(idle);
     ds.nfacets = int64_t(nact);
     ds.ntwo = int64_t(ntwo);
-    ds.cap = 0;
-    reserve_split(ds, 1);
+    split_slots(ds, 1);
 }
 
 bool Operator::poisson_mfma_compiled() const {
@@ -1816,13 +1819,13 @@ template <class T> void Operator::dispatch(T const* x, T* y, int ncols, int64_t 
             if constexpr (std::is_same<T, double>::value) return *m64_;
             else return *m32_;
         }();
-        reserve_split(ds, ncols);
+        T* const slots = split_slots(ds, ncols);
         const int64_t ldL = int64_t(E_) * (D_ + 1) * int64_t(block_size());
         const int p = sizeof(T) == 8 ? 0 : 1;
         SplitArgs<T> sa = split_args(dm, ds);
         sa.xcd_remap = split_xcd_[p];
         sa.small = split_small_bits(int(sizeof(T)), ncols);
-        TDG_HIP(launch_elasticity_split<T>(D_, N_, split_shape_[p], sa, x, y, ds.L.ptr, ncols, ncols > 1 ? ld : 0,
+        TDG_HIP(launch_elasticity_split<T>(D_, N_, split_shape_[p], sa, x, y, slots, ncols, ncols > 1 ? ld : 0,
                                            ldL, stream_));
     } else if (uses_mfma()) {
         if constexpr (std::is_same<T, double>::value) launch_mfma(*m64_, x, y, ncols, ld);

@@ -57,13 +57,14 @@ template <class T> struct DeviceMfma {
 };
 
 // Facet records, penalties and facet info of the two-kernel (facet + element) MFMA apply, and the
-// buffer of lifted facet contributions per element face (cap columns; cleared when allocated, so the
-// slots of faces without a facet term stay zero).
+// lifted facet contributions per element face (cleared when allocated, so the slots of faces without a
+// facet term stay zero): one column's, which stay where they are (a captured apply replays into them), and
+// those of a batch (cap columns, replaced by larger ones).
 template <class T> struct DeviceSplit {
     DeviceArray<T> FR, FPen;
     DeviceArray<int32_t> FInfo; // int4 per facet
     DeviceArray<int32_t> idle;  // slots (element * (D+1) + face) of faces without a facet term
-    DeviceArray<T> L;
+    DeviceArray<T> L, LB;
     int64_t nfacets = 0, ntwo = 0;
     int cap = 0;
 };
@@ -280,7 +281,7 @@ private:
     template <class T> void upload_mfma_faces(DeviceMfma<T>& d);
     template <class T> void upload_split(DeviceSplit<T>& d);
     template <class T> SplitArgs<T> split_args(DeviceMfma<T> const& m, DeviceSplit<T> const& s) const;
-    template <class T> void reserve_split(DeviceSplit<T>& s, int ncols);
+    template <class T> T* split_slots(DeviceSplit<T>& s, int ncols);
     // whether an apply of ncols columns in pb bytes a real takes the matrix-core Poisson kernels (by size; by
     // operator: whether they are compiled for it)
     bool poisson_mfma_compiled() const;

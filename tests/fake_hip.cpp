@@ -154,10 +154,11 @@ void __hipUnregisterFatBinary(void**) {}
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 hipError_t hipLaunchKernel(void const* f, dim3 g, dim3 b, void** args, size_t, hipStream_t s) {
     std::string const& n = g_names[f];
-    // the trace buffer is the third argument of both Poisson kernels
-    const bool poisson = n.find("poisson_trace") != n.npos || n.find("poisson_element") != n.npos;
-    log("launch %s grid %ux%u block %u stream %p traces %p", n.c_str(), g.x, g.y, b.x, (void*)s,
-        poisson ? *static_cast<void**>(args[2]) : nullptr);
+    // the buffer between the two kernels (facet slots, traces) is the third argument of all four
+    const bool two = n.find("poisson_trace") != n.npos || n.find("poisson_element") != n.npos ||
+                     n.find("elasticity_facet_kernel") != n.npos || n.find("elasticity_element_kernel") != n.npos;
+    log("launch %s grid %ux%u block %u stream %p between %p", n.c_str(), g.x, g.y, b.x, (void*)s,
+        two ? *static_cast<void**>(args[2]) : nullptr);
     return hipSuccess;
 }
 }

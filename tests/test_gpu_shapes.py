@@ -218,13 +218,14 @@ def test_poisson_column_ranges(cuda):
         assert torch.equal(y, Y[k])
 
 
-@pytest.mark.parametrize("D,n,N", [(2, (65, 63), 4), (3, (11, 10, 10), 2)])
-def test_poisson_captured_and_on_two_streams(cuda, D, n, N):
-    """The matrix-core Poisson apply captured into a graph and replayed after a larger batch, with eager
-    applies between, and applies of two vectors queued on two streams in turn: the eager results' bits."""
+@pytest.mark.parametrize("kind,D,n,N", [(1, 2, (65, 63), 4), (1, 3, (11, 10, 10), 2), (0, 3, (4, 3, 3), 3)])
+def test_captured_and_on_two_streams(cuda, kind, D, n, N):
+    """The matrix-core Poisson apply and the two-kernel apply captured into a graph and replayed after a larger
+    batch, with eager applies between, and applies of two vectors queued on two streams in turn: the eager
+    results' bits."""
     import torch
 
-    c = Mixed(D, n, N, kind=1, seed=3)
+    c = Mixed(D, n, N, kind=kind, seed=3)
     c.op.upload()
     X = torch.rand((5, c.n), dtype=torch.float64, device=cuda)
     ref = torch.empty_like(X)

@@ -39,6 +39,9 @@ BATCH = {8: lib().tdg_mult_batched, 4: lib().tdg_mult_batched_f32}
 
 def traces(lines):
     return {l.split()[-1] for l in lines if "poisson_trace" in l or "poisson_element" in l}
+
+def slots(lines):
+    return {l.split()[-1] for l in lines if "facet_kernel" in l or "element_kernel" in l}
 """
 
 
@@ -57,18 +60,23 @@ def host_hip(tmp_path_factory):
 
 
 def test_batch_that_finds_no_memory_leaves_single_applies_whole(host_hip):
-    """A column count whose facet slots do not fit is an error; the one-column apply after it allocates its
-    slots again instead of writing through the lost buffer."""
+    """A column count whose facet slots do not fit is an error; the applies after it write slots that are
+    there, not the lost buffer."""
     host_hip("""
 op = operator(0, 3, 2, 4)
 for pb in (8, 4):
     assert MULT[pb](op._h, X, Y) == 0
+    one = slots(log())
+    assert BATCH[pb](op._h, X, Y, 2, op.n) == 0
     F.fake_room(1 << 22)
     assert BATCH[pb](op._h, X, Y, 64, op.n) == -3 and b"out of memory" in lib().tdg_last_error()
     F.fake_room(1 << 40)
     log()
-    assert MULT[pb](op._h, X, Y) == 0
-    assert any(int(l.split()[2]) == op.n * 4 * pb for l in log("^malloc")), "slots of one column"
+    assert MULT[pb](op._h, X, Y) == 0 and slots(log()) == one
+    assert BATCH[pb](op._h, X, Y, 2, op.n) == 0
+    lines = log()
+    (m,) = [l.split() for l in lines if l.startswith("malloc")]
+    assert int(m[2]) == 2 * op.n * 4 * pb and slots(lines) == {m[1]}
 """)
 
 
@@ -348,3 +356,24 @@ for D, n, N, mfma in ((3, 1, 4, False), (3, 4, 4, False), (3, 5, 4, True), (3, 1
     assert ("mfma" in l) == mfma, (D, n, N, l)
     assert mfma or "grid %dx1" % op.E in l
 """)
+
+
+@pytest.mark.parametrize("pb", [8, 4])
+@pytest.mark.parametrize("D,n,N", [(3, 2, 4), (2, 9, 6)])
+def test_single_column_slots_stay_in_place(host_hip, D, n, N, pb):
+    """A batch of any size leaves the facet slots of single applies where they are (a captured single apply
+    replays into them)."""
+    host_hip("""
+D, n, N, pb = %r
+op = operator(0, D, n, N)
+op.upload()
+assert MULT[pb](op._h, X, Y) == 0
+one = slots(log())
+assert len(one) == 1
+for cols in (2, 5, 3, 40):
+    assert BATCH[pb](op._h, X, Y, cols, op.n) == 0
+    lines = log()
+    assert not one & slots(lines) and not [l for l in lines if l.startswith("free") and l.split()[1] in one]
+    assert MULT[pb](op._h, X, Y) == 0
+    assert slots(log()) == one
+""" % ((D, n, N, pb),))
